@@ -63,7 +63,11 @@ template <int BITS, int G>
 struct Geo {
   static constexpr int STEPS = G / 32;                  // instructions (per part) per group
   static constexpr int W = G * BITS / 32;               // u32 words of one group of one row
-  static constexpr int LDI = W % 4 == 0 ? W / 4 : (W % 2 == 0 ? W / 2 : W);   // load instructions per group
+  // Load instructions per group, at least: the compiler joins load_words' 8- and 4-byte
+  // loads into 16-byte ones (six words: two instructions).  The waits that leave the codes
+  // in flight count by this; counted as written (three for six words), they let the last
+  // scale runs of a 3-bit bank still be on their way when the items read them.
+  static constexpr int LDI = (W + 3) / 4;
 };
 
 // The W words of one group of one row (16-, 8- or 4-byte loads as the group's

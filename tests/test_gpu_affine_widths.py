@@ -287,3 +287,25 @@ def test_affine_prefill_config3_routing(cuda, bits, group, monkeypatch):
         rows_of[e] = np.asarray([i for i, (a, c) in enumerate(rows.tolist()) if (a, c) in want])
     _grouped_check(f"config3 routing prefill {bits}-bit g{group}", fmt, 0, _f32(x), oi, ow, _np(routed), _f32(out),
                    _f32(y), E, rows_of=rows_of)
+
+
+@pytest.mark.parametrize("bits,group", [(3, 64), (3, 32), (4, 64)])
+def test_affine_decode_repeats_exactly(cuda, bits, group):
+    """Given experts of six layers in turn (no layer's bytes stay in cache), 40 rounds: every round
+    gives the first one's bits, so no item reads a scale run before its copy has landed."""
+    from cachalot_amd import synth
+    from cachalot_amd.moe_decode import decode_experts
+
+    fmt = _fmt(bits, group, "float16")
+    store = make_store(fmt, n_layers=6, n_experts=64)
+    idx = torch.tensor([5, 37, 60, 12, 50, 19], dtype=torch.int32, device=cuda)
+    w = torch.full((6,), 1 / 6, dtype=torch.float32, device=cuda)
+    x = synth.activations(SEED, 3700, 1, 4096, cuda)[0]
+
+    def one(la):
+        return decode_experts(x, store.pool, store.layer_table(la), idx, w, want_out=False)[0].clone()
+
+    first = [one(la) for la in range(6)]
+    for _ in range(40):
+        for la in range(6):
+            assert torch.equal(one(la), first[la])
