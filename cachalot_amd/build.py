@@ -36,9 +36,10 @@ CFLAGS = [
 ]
 
 
-# Per-file flags.  prefill_affine_mx.hip: matrix-core results in VGPRs, where its
-# per-group fold reads them (the other kernels keep their accumulators in AGPRs).
-FILE_FLAGS = {"prefill_affine_mx.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]}
+# Per-file flags.  prefill_affine_mx.hip, small_rows_mx.hip: matrix-core results in VGPRs,
+# where their per-group folds read them (the other kernels keep their accumulators in AGPRs).
+_VGPR_TILES = ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]
+FILE_FLAGS = {"prefill_affine_mx.hip": _VGPR_TILES, "small_rows_mx.hip": _VGPR_TILES}
 
 
 def sources() -> list[Path]:

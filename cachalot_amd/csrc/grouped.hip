@@ -70,6 +70,15 @@ int launch_prefill_mx(const uint16_t* x, int T, const uint8_t* pool, const decod
                       int max_tiles, const int32_t* row_token, const int32_t* row_slot, const float* row_w, int D,
                       int F, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s);
 bool prefill_mx_q2_supported(int D, int F, const decode::Layout& L);
+// few rows per expert on the block-scaled matrix cores (small_rows_mx.hip, prefill_mx.hip);
+// bits 0: FP4
+int small_rows_mt(int ak);
+int small_rows_ak(int bits, int group);
+bool small_rows_supported(int ak, int D, int F, const decode::Layout& L);
+int launch_prefill_small(int bits, int group, const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
+                         const int4* recs, const int32_t* recs_n, const int32_t* row_token,
+                         const int32_t* row_slot, const float* row_w, int D, int F, int k, float limit, uint8_t* ws,
+                         uint16_t* y, hipStream_t s);
 int launch_prefill_mx_q2(const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
                          const int32_t* slot_table, const int32_t* offsets, const int2* tiles,
                          const int32_t* tiles_n, int max_tiles, const int32_t* row_token, const int32_t* row_slot,
@@ -236,6 +245,32 @@ __global__ void __launch_bounds__(1024) tile_list_kernel(const int32_t* __restri
   const int first = sc[e] - cnt;
   if (e == 1023) tiles_n[0] = sc[1023];
   for (int t = 0; t < cnt; ++t) tiles[first + t] = make_int2(e, offsets[e] + t * MT);
+}
+
+// The same tiles as records (expert, first row, end row, slot) for the few-row kernels.
+__global__ void __launch_bounds__(1024) tile_recs_kernel(const int32_t* __restrict__ offsets,
+                                                         const int32_t* __restrict__ slot_table, int E, int MT,
+                                                         int4* __restrict__ recs, int32_t* __restrict__ recs_n) {
+  __shared__ int sc[1024];
+  const int e = threadIdx.x;
+  int cnt = 0, r0 = 0, r1 = 0, slot = -1;
+  if (e < E) {
+    r0 = offsets[e];
+    r1 = offsets[e + 1];
+    slot = slot_table[e];
+    cnt = r1 > r0 ? 1 + (r1 - r0 - 1) / MT : 0;
+  }
+  sc[e] = cnt;
+  __syncthreads();
+  for (int off = 1; off < 1024; off *= 2) {
+    const int v = e >= off ? sc[e - off] : 0;
+    __syncthreads();
+    sc[e] += v;
+    __syncthreads();
+  }
+  const int first = sc[e] - cnt;
+  if (e == 1023) recs_n[0] = sc[1023];
+  for (int t = 0; t < cnt; ++t) recs[first + t] = make_int4(e, r0 + t * MT, min(r1, r0 + (t + 1) * MT), slot);
 }
 
 // ------------------------------------------------------------ grouped GEMM ---
@@ -979,11 +1014,12 @@ struct GroupedWs {
 inline GroupedWs grouped_ws(int T, int k, int E, int D, int F) {
   GroupedWs w;
   const int rows = T * k;
-  w.max_tiles = rows / 16 + std::min(E, rows) + 1;   // bound for MT >= 16
+  w.max_tiles = rows / 4 + std::min(E, rows) + 1;   // bound for MT >= 4
   w.tiles_n = 0;
   w.tiles = 256;
-  // int2 tiles, or one int4 record per active expert (matrix-core batched decode)
-  w.hidden = w.tiles + align256(std::max((size_t)w.max_tiles * sizeof(int2), (size_t)std::min(E, rows) * sizeof(int4)));
+  // int2 tiles, or int4 records (few-row kernels: one per tile; matrix-core batched decode:
+  // one per active expert)
+  w.hidden = w.tiles + align256((size_t)w.max_tiles * sizeof(int4));
   const size_t hid = std::max((size_t)rows * F * sizeof(uint16_t), (size_t)rows * ((F + 127) / 128) * 320);
   w.xplanes = w.hidden + align256(hid);
   w.mx = w.xplanes + align256((size_t)T * ((D + 127) / 128) * 320);
@@ -1027,6 +1063,22 @@ inline bool prefill_bf16_requested() {
   return env && env[0] == '1';
 }
 
+// Where the few-row weight stream (small_rows_mx.hip) is the faster one, in routes per
+// expert.  It reads an expert's weights once per 8 (4) rows, the 64-row tiles once per 64
+// but at a lower rate while tiles are nearly empty.  Per layer at D 4096 x F 2880, 384
+// experts top-6, against the path on the other side of the line, us:
+//   FP4: 200 tokens (3.1 per expert) 1366 against 1745 (bf16-MFMA 16-row tiles), 400
+//     (6.3) 1884 against 1752 (64-row tiles): up to 5;
+//   3-bit g64: 200 tokens 1940 against 5926 (bf16-MFMA), 256 2400 against 2650 (64-row), 400
+//     3300 against 2720: up to 4, the same for the other widths and groups;
+//   2-bit g128: 64 tokens (1 per expert) 573 against 535 (one-token items per row), 128 (2)
+//     848 against 918, 400 1440 against 1703 (64-row), 600 (9.4) 2050 against 1850: 1.5 to 8.
+inline bool small_rows_wanted(int kind, int rows, int E) {
+  if (kind == KIND_FP4) return rows < 5 * E;
+  if (kind == KIND_Q2) return 2 * rows >= 3 * E && rows < 8 * E;
+  return rows < 4 * E;
+}
+
 template <int KIND>
 int launch_grouped(const uint16_t* x, const uint8_t* pool, const cachalot_expert_layout* layout,
                    const int32_t* slot_table, const int32_t* offsets, const int32_t* row_token,
@@ -1062,7 +1114,13 @@ int launch_grouped(const uint16_t* x, const uint8_t* pool, const cachalot_expert
   // tiles of 64 rows when experts see many tokens, 16 for batched decode
   const int MT = T * k >= 4 * E ? 64 : 16;
   uint32_t* zeros = reinterpret_cast<uint32_t*>(ws + wo.tiles_n + 128);
-  const bool batched = KIND == KIND_Q2 && MT == 16 && q2mx_supported(D, F, k) && !small_tiles_requested();
+  // few rows per expert: the weight stream of small_rows_mx.hip
+  constexpr int SBITS = KIND == KIND_FP4 ? 0 : KIND == KIND_Q2 ? 2 : aff_bits(KIND);
+  constexpr int SGROUP = is_aff(KIND) ? aff_group(KIND) : KC;
+  const int sak = small_rows_ak(SBITS, SGROUP), smt = small_rows_mt(sak);
+  const bool small = small_rows_wanted(KIND, T * k, E) && small_rows_supported(sak, D, F, L) &&
+                     !small_tiles_requested() && !prefill_bf16_requested();
+  const bool batched = KIND == KIND_Q2 && MT == 16 && q2mx_supported(D, F, k) && !small && !small_tiles_requested();
   // routes given: permuted by the batched prep launch when one workgroup holds them, else here
   const bool fused = ridx != nullptr && batched && T * k <= PERMUTE_THREADS;
   if (ridx != nullptr && !fused) {
@@ -1080,6 +1138,14 @@ int launch_grouped(const uint16_t* x, const uint8_t* pool, const cachalot_expert
   hipLaunchKernelGGL(drop_zero_kernel, dim3(16), dim3(256), 0, s, offsets, E, T * k, T, k, D, row_token, row_slot, y);
   rc = check_launch("drop_zero_kernel");
   if (rc) return rc;
+  if (small) {
+    int4* recs = reinterpret_cast<int4*>(ws + wo.tiles);
+    hipLaunchKernelGGL(tile_recs_kernel, dim3(1), dim3(1024), 0, s, offsets, slot_table, E, smt, recs, tiles_n);
+    rc = check_launch("tile_recs_kernel");
+    if (rc) return rc;
+    return launch_prefill_small(SBITS, SGROUP, x, T, pool, L, recs, tiles_n, row_token, row_slot, row_w,
+                                D, F, k, limit, ws + wo.mx, y, s);
+  }
   const int max_tiles = (T * k) / MT + std::min(E, T * k) + 1;
   if (KIND == KIND_FP4 && MT == 64 && prefill_mx_supported(D, F, L) && !small_tiles_requested() &&
       !prefill_bf16_requested() && max_tiles <= (1 << 20)) {

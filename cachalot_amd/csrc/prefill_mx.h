@@ -63,9 +63,31 @@ struct MxArgs {
   uint16_t* y;                // down: [T, k, N]
   const float* asum;          // 2-bit: chunk sums of the A source rows [source rows][kch]
   float* hsum;                // 2-bit gate/up: chunk sums of h [rows][hkch]
+  const int4* recs;           // few-row kernels: the tiles as (expert, first row, end row, slot)
 };
 
 __host__ __device__ inline int scale_row_bytes(int K) { return (K / 32 * 2 + 15) / 16 * 16; }
+
+// Position along K of element n of a 32-element block in the planes of the few-row
+// kernels (small_rows_mx.hip), the order its BITS-bit codes spread to fp4 in: 2-bit even
+// elements of each 16, then odd; 3-bit code 4t + r at 3t + r (r < 3), codes 4t + 3 in the
+// last eight; others natural.
+template <int BITS>
+__host__ __device__ inline int plane_pos(int n) {
+  if (BITS == 2) return (n & 16) + ((n & 1) ? 8 + ((n & 15) >> 1) : (n & 15) >> 1);
+  if (BITS == 3) {
+    const int t = n >> 2, r = n & 3;
+    return r < 3 ? 3 * t + r : 24 + ((0x65274130 >> (4 * t)) & 15);
+  }
+  return n;
+}
+
+// Place of 32-element block b of a 128-element chunk in those planes (its own inverse):
+// the 2-bit codes reach the lane groups in the order 0, 2, 1, 3.
+template <int BITS>
+__host__ __device__ inline int block_at(int b) {
+  return BITS == 2 && (b == 1 || b == 2) ? 3 - b : b;
+}
 
 // Plane scale exponent of a block whose largest magnitude is m: E = e(m) - 7,
 // clamped so that both E8M0 bytes (E + 127, E + 123) are finite scales.
