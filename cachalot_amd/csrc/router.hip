@@ -20,6 +20,8 @@
 //                         are loaded once per wave and reused for TT tokens.
 //   router_topk_kernel    one wave per token; k rounds of a wave-wide argmax
 //                         under the order's total order (value, then index).
+#include <algorithm>
+
 #include "mx_tile.h"
 #include "router_launch.h"
 #include "router_math.h"
@@ -99,30 +101,32 @@ __global__ void __launch_bounds__(64) router_topk_kernel(const float* __restrict
   if (threadIdx.x == 0) normalise_weights(top_v, k, route_scale, norm, w + (size_t)t * k);
 }
 
-// Many tokens: one 256-thread workgroup = 64 tokens x 32 experts, each thread 4
-// tokens (tq + 16 a) x 2 experts (eq + 16 b).  The same arithmetic as router_row:
-// chunk c (of 64) of every dot product is a sequential fp32 sum of its D/64
-// products in k order, and the 64 chunk sums meet in the pairwise tree (left +
-// right) the xor butterfly forms, kept as a binary-counter stack of six partial
-// nodes per dot product.  Chunk by chunk, the x and W slices are staged in LDS as
-// bf16 (double-buffered, one barrier per chunk) and read as 8-value runs (one
-// 16-byte read per token or expert feeds 8 x 4 products); rows are padded to an
-// odd number of 16-byte slots so the 16 experts a wave row reads hit distinct
-// bank groups.  fma(x, w, s) equals s + x * w here: the product of two bf16
-// values is exact in fp32 (16 significant bits) unless it is below 2^-133.
-constexpr int RT_TA = 4;             // tokens per thread (tq + 16 a)
+// Many tokens: one workgroup = 16 TA tokens x 32 experts, each thread TA tokens (tq + 16
+// a) x 2 experts (eq + 16 b).  The same arithmetic as router_row: chunk c (of 64) of every
+// dot product is a sequential fp32 sum of its D/64 products in k order, and the 64 chunk
+// sums meet in the pairwise tree (left + right) the xor butterfly forms, kept as a
+// binary-counter stack of partial nodes per dot product.  Chunk by chunk, the x and W
+// slices are staged in LDS as bf16 (double-buffered, one barrier per chunk) and read as
+// 8-value runs (one 16-byte read per token or expert feeds 8 x 2 TA products); rows are
+// padded to an odd number of 16-byte slots so the 16 experts a wave row reads hit distinct
+// bank groups.  fma(x, w, s) equals s + x * w here: the product of two bf16 values is
+// exact in fp32 (16 significant bits) unless it is below 2^-133.
+//
+// SP: the chunks are dealt to SP groups of 256 threads, a run of 64 / SP each (a subtree of
+// the pairwise sum), whose roots meet at the end.  What bounds the kernel is the fp32
+// multiply-adds, so it wants every SIMD busy: 64 tokens x 32 experts with SP = 1 does that
+// from some 2300 tokens on (768 workgroups at 4096 tokens x 384 experts), SP = 4 below.
 constexpr int RT_TB = 2;             // experts per thread (eq + 16 b)
-constexpr int RT_T = 16 * RT_TA;     // tokens per workgroup
 constexpr int RT_E = 16 * RT_TB;     // experts per workgroup
 constexpr int RT_MAXCH = 80;         // D / 64 <= 80 (D <= 5120)
-constexpr int RT_MAXS = RT_MAXCH * 2 + 32;   // staged row bytes, padding included
-constexpr int RT_MIN_T = 1024;       // fewer tokens: the 4-token kernel fills the chip better
+
+constexpr int64_t RT_MIN_DOTS = 160 * 384;   // scores
 
 __host__ __device__ inline int rt_stride(int ch) { return ch * 2 + ((ch / 8) % 2 == 0 ? 16 : 32); }
 
 // Chunk c of a tile's x rows, then its W rows, as 16-byte items (rows past T / E:
 // clamped, unused), and the store of those items into a staged buffer.
-template <int N>
+template <int N, int TT>
 __device__ __forceinline__ void rt_load(uint4 (&v)[N], const uint16_t* __restrict__ x, const uint16_t* __restrict__ W,
                                         int T, int D, int E, int t0, int e0, int c, int tid, int items, int per_row) {
   const int ch = 8 * per_row;
@@ -130,7 +134,7 @@ __device__ __forceinline__ void rt_load(uint4 (&v)[N], const uint16_t* __restric
   for (int j = 0; j < N; ++j) {
     const int it = min(tid + 256 * j, items - 1);
     const int r = it / per_row, q = it - r * per_row;
-    const uint16_t* src = r < RT_T ? x + (size_t)min(t0 + r, T - 1) * D : W + (size_t)min(e0 + r - RT_T, E - 1) * D;
+    const uint16_t* src = r < TT ? x + (size_t)min(t0 + r, T - 1) * D : W + (size_t)min(e0 + r - TT, E - 1) * D;
     v[j] = *reinterpret_cast<const uint4*>(src + c * ch + 8 * q);
   }
 }
@@ -145,44 +149,54 @@ __device__ __forceinline__ void rt_store(uint8_t* buf, const uint4 (&v)[N], int 
   }
 }
 
-__global__ void __launch_bounds__(256) router_tiled_kernel(const uint16_t* __restrict__ x,
-                                                           const uint16_t* __restrict__ W, int T, int D, int E,
-                                                           float gate_temp, int fn, float* __restrict__ scores) {
-  __shared__ __align__(16) uint8_t st[2][(RT_T + RT_E) * RT_MAXS];
-  const int tid = threadIdx.x;
+// dynamic LDS = SP * 2 * (16 TA + RT_E) * rt_stride(D / 64)
+template <int TA, int SP>
+__global__ void __launch_bounds__(256 * SP) router_tiled_kernel(const uint16_t* __restrict__ x,
+                                                                const uint16_t* __restrict__ W, int T, int D, int E,
+                                                                float gate_temp, int fn,
+                                                                float* __restrict__ scores) {
+  constexpr int TT = 16 * TA;                 // tokens per workgroup
+  constexpr int NC = CHUNKS / SP;             // chunks per group
+  constexpr int LEV = NC == 64 ? 6 : 4;       // levels of a group's subtree
+  static_assert(NC == 64 || NC == 16, "SP is 1 or 4");
+  extern __shared__ __align__(16) uint8_t rt_lds[];
+  const int grp = SP == 1 ? 0 : threadIdx.x >> 8;
+  const int tid = threadIdx.x & 255;
   const int eq = tid & 15, tq = tid >> 4;
-  const int t0 = blockIdx.x * RT_T, e0 = blockIdx.y * RT_E;
+  const int t0 = blockIdx.x * TT, e0 = blockIdx.y * RT_E;
   const int per_row = D / 512;                // 16-byte items per staged row
   const int ch = 8 * per_row;                 // D / 64
   const int S = rt_stride(ch);
-  const int items = (RT_T + RT_E) * per_row;  // x rows first, then W rows
-  constexpr int MAXIT = ((RT_T + RT_E) * RT_MAXCH / 8 + 255) / 256;
+  const int items = (TT + RT_E) * per_row;    // x rows first, then W rows
+  constexpr int MAXIT = ((TT + RT_E) * RT_MAXCH / 8 + 255) / 256;
+  uint8_t* st = rt_lds + grp * 2 * (TT + RT_E) * S;
+  const int c0 = grp * NC;
 
-  float stk[6][RT_TA * RT_TB];
-  float node[RT_TA * RT_TB];
+  float stk[LEV][TA * RT_TB];
+  float node[TA * RT_TB];
   uint4 v[MAXIT];
-  rt_load(v, x, W, T, D, E, t0, e0, 0, tid, items, per_row);
-  rt_store(st[0], v, tid, items, per_row, S);
+  rt_load<MAXIT, TT>(v, x, W, T, D, E, t0, e0, c0, tid, items, per_row);
+  rt_store(st, v, tid, items, per_row, S);
   __syncthreads();
-  for (int c = 0; c < CHUNKS; ++c) {
-    if (c + 1 < CHUNKS) rt_load(v, x, W, T, D, E, t0, e0, c + 1, tid, items, per_row);
-    const uint8_t* buf = st[c & 1];
-    float acc[RT_TA * RT_TB];
+  for (int c = 0; c < NC; ++c) {
+    if (c + 1 < NC) rt_load<MAXIT, TT>(v, x, W, T, D, E, t0, e0, c0 + c + 1, tid, items, per_row);
+    const uint8_t* buf = st + (c & 1) * (TT + RT_E) * S;
+    float acc[TA * RT_TB];
 #pragma unroll
-    for (int p = 0; p < RT_TA * RT_TB; ++p) acc[p] = 0.0f;
+    for (int p = 0; p < TA * RT_TB; ++p) acc[p] = 0.0f;
     // (a runtime loop: unrolled, the scheduled-ahead reads push the kernel to one wave per SIMD)
     for (int k8 = 0; k8 < per_row; ++k8) {
-      uint4 xa[RT_TA], wb[RT_TB];
+      uint4 xa[TA], wb[RT_TB];
 #pragma unroll
-      for (int a = 0; a < RT_TA; ++a) xa[a] = *reinterpret_cast<const uint4*>(buf + (tq + 16 * a) * S + 16 * k8);
+      for (int a = 0; a < TA; ++a) xa[a] = *reinterpret_cast<const uint4*>(buf + (tq + 16 * a) * S + 16 * k8);
 #pragma unroll
       for (int b = 0; b < RT_TB; ++b)
-        wb[b] = *reinterpret_cast<const uint4*>(buf + (RT_T + eq + 16 * b) * S + 16 * k8);
+        wb[b] = *reinterpret_cast<const uint4*>(buf + (TT + eq + 16 * b) * S + 16 * k8);
 #pragma unroll
       for (int h = 0; h < 4; ++h) {            // the 8 values in k order: word h, low then high half
-        float xl[RT_TA], xh[RT_TA], wl[RT_TB], wh[RT_TB];
+        float xl[TA], xh[TA], wl[RT_TB], wh[RT_TB];
 #pragma unroll
-        for (int a = 0; a < RT_TA; ++a) {
+        for (int a = 0; a < TA; ++a) {
           const uint32_t u = h == 0 ? xa[a].x : h == 1 ? xa[a].y : h == 2 ? xa[a].z : xa[a].w;
           xl[a] = __uint_as_float(u << 16);
           xh[a] = __uint_as_float(u & 0xffff0000u);
@@ -194,7 +208,7 @@ __global__ void __launch_bounds__(256) router_tiled_kernel(const uint16_t* __res
           wh[b] = __uint_as_float(u & 0xffff0000u);
         }
 #pragma unroll
-        for (int a = 0; a < RT_TA; ++a)
+        for (int a = 0; a < TA; ++a)
 #pragma unroll
           for (int b = 0; b < RT_TB; ++b) {
             float t = acc[RT_TB * a + b];
@@ -204,27 +218,40 @@ __global__ void __launch_bounds__(256) router_tiled_kernel(const uint16_t* __res
           }
       }
     }
-    if (c + 1 < CHUNKS) rt_store(st[(c + 1) & 1], v, tid, items, per_row, S);
+    if (c + 1 < NC) rt_store(st + ((c + 1) & 1) * (TT + RT_E) * S, v, tid, items, per_row, S);
     // merge chunk c into the tree (c is uniform: every branch below is too)
 #pragma unroll
-    for (int p = 0; p < RT_TA * RT_TB; ++p) node[p] = acc[p];
+    for (int p = 0; p < TA * RT_TB; ++p) node[p] = acc[p];
     // chunk c closes the nodes of the levels below its lowest zero bit
-    const int up = __builtin_ctz(~c);   // levels merged (6 after the last chunk)
+    const int up = __builtin_ctz(~c);   // levels merged (LEV after the last chunk)
 #pragma unroll
-    for (int L = 0; L < 6; ++L) {
+    for (int L = 0; L < LEV; ++L) {
       if (L < up) {
 #pragma unroll
-        for (int p = 0; p < RT_TA * RT_TB; ++p) node[p] = stk[L][p] + node[p];
+        for (int p = 0; p < TA * RT_TB; ++p) node[p] = stk[L][p] + node[p];
       } else if (L == up) {
 #pragma unroll
-        for (int p = 0; p < RT_TA * RT_TB; ++p) stk[L][p] = node[p];
+        for (int p = 0; p < TA * RT_TB; ++p) stk[L][p] = node[p];
       }
     }
     __syncthreads();
   }
-  // after chunk 63 every level merged: node holds the root
+  // after the last chunk every level merged: node holds the group's root
+  if constexpr (SP == 4) {   // (g0 + g1) + (g2 + g3), by group 0 (the staging is done with)
+    float* roots = reinterpret_cast<float*>(rt_lds);   // [group][dot][thread]
 #pragma unroll
-  for (int a = 0; a < RT_TA; ++a) {
+    for (int p = 0; p < TA * RT_TB; ++p) roots[(grp * TA * RT_TB + p) * 256 + tid] = node[p];
+    __syncthreads();
+    if (grp != 0) return;
+#pragma unroll
+    for (int p = 0; p < TA * RT_TB; ++p) {
+      const float* r = roots + p * 256 + tid;
+      constexpr int G = TA * RT_TB * 256;
+      node[p] = (r[0] + r[G]) + (r[2 * G] + r[3 * G]);
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < TA; ++a) {
     const int t = t0 + tq + 16 * a;
     if (t >= T) continue;
 #pragma unroll
@@ -233,6 +260,20 @@ __global__ void __launch_bounds__(256) router_tiled_kernel(const uint16_t* __res
       if (e < E) scores[(size_t)t * E + e] = score_of(node[RT_TB * a + b] / gate_temp, fn);
     }
   }
+}
+
+template <int TA, int SP>
+int launch_tiled(const uint16_t* x, const uint16_t* W, int T, int D, int E, float gate_temp, int fn, float* scores,
+                 hipStream_t s) {
+  const size_t lds = (size_t)SP * std::max((size_t)2 * (16 * TA + RT_E) * rt_stride(D / CHUNKS),
+                                           SP == 1 ? (size_t)0 : (size_t)TA * RT_TB * 256 * 4);
+  auto k = router_tiled_kernel<TA, SP>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
+      hipSuccess)
+    return fail(CACHALOT_EHIP, "router: cannot grant %zu bytes of LDS", lds);
+  hipLaunchKernelGGL(k, dim3((T + 16 * TA - 1) / (16 * TA), (E + RT_E - 1) / RT_E), dim3(256 * SP), lds, s, x, W, T, D,
+                     E, gate_temp, fn, scores);
+  return check_launch("router_tiled_kernel");
 }
 
 }  // namespace
@@ -254,11 +295,20 @@ static void launch_scores_tt(const uint16_t* x, const uint16_t* W, int T, int D,
 int launch_router_scores(const uint16_t* x, const uint16_t* W, int T, int D, int E, float gate_temp, int fn,
                          float* scores, hipStream_t s, const decode::RouteTail* tail, uint8_t* xplanes) {
   decode::RouteTail none{};
-  // the tiled kernel needs enough tiles to fill the chip (32 x 64 per workgroup)
-  if (T >= RT_MIN_T && D % 512 == 0 && D / CHUNKS <= RT_MAXCH) {
-    hipLaunchKernelGGL(router_tiled_kernel, dim3((T + RT_T - 1) / RT_T, (E + RT_E - 1) / RT_E), dim3(256), 0, s, x,
-                       W, T, D, E, gate_temp, fn, scores);
-    return check_launch("router_tiled_kernel");
+  // The tiled kernel from RT_MIN_DOTS scores on (384 experts: 160 tokens; 200 tokens 91 us
+  // on the 4-token kernel against 56, 1000 tokens 417 against 127).  Below four chip-filling
+  // rounds of 32 x 32 tiles the chunks are split over four groups of threads; of 16, 32 and
+  // 64 tokens per tile the fewest rounds, weighed by what a round of each takes (52, 71 and
+  // 117 us at D = 4096), win (1500 tokens: 186 us with 32, 214 with 16, 242 with 64, 262
+  // unsplit; 4096: 324 unsplit, 381 with 32).
+  if ((int64_t)T * E >= RT_MIN_DOTS && D % 512 == 0 && D / CHUNKS <= RT_MAXCH) {
+    const int et = (E + RT_E - 1) / RT_E;
+    auto rounds = [&](int tokens) { return ((int64_t)((T + tokens - 1) / tokens) * et + 255) / 256; };
+    if (rounds(32) >= 4) return launch_tiled<4, 1>(x, W, T, D, E, gate_temp, fn, scores, s);
+    const int64_t c16 = 52 * rounds(16), c32 = 71 * rounds(32), c64 = 117 * rounds(64);
+    if (c16 <= c32 && c16 <= c64) return launch_tiled<1, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
+    if (c32 <= c64) return launch_tiled<2, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
+    return launch_tiled<4, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
   }
   // tokens per wave: 4 from 8 tokens on, 2 below (twice the waves for a small batch:
   // B = 4 68.4 against 70 us per batched step; at B = 32, 2 per wave lost 2.6 us)
