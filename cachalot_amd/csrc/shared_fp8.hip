@@ -242,30 +242,41 @@ int launch_quant(const uint16_t* x, int ldx, int M, int K, bool swiglu, float li
 }
 
 // ------------------------------------------------------------ many-token GEMM ---
-// One 512-thread workgroup = a 128-token x 256-row tile of one matrix; wave (wm, wn),
-// wm < 2, wn < 4, owns tokens [64 wm, +64) x rows [64 wn, +64) as 4 x 4 tiles of
-// 16 x 16.  K runs in stages of one 32-element block (one E8M0 scale per row and
-// stage).  The tiles stay E4M3 bytes in LDS (rows 40 bytes apart, so the 16 rows of a
-// fragment fall on distinct banks) with their scale bytes beside them; a wave converts
-// each fragment as it reads it (8 values per lane, scale folded in: exact) for
-// v_mfma_f32_16x16x32_bf16.  Two LDS buffers, GM_RING blocks of bytes in registers
-// (the loads run that many blocks ahead); 123 VGPRs, four waves per SIMD.  Rows past
-// M and N read row 0 (masked at the store).
-// Measured at M = 4096 (the whole expert, ~450 us against 620 us for 64 x 64 tiles
-// read straight from global memory): bf16 tiles in LDS, 64 x 128 wave tiles, two
-// waves per SIMD and one to three blocks of prefetch all landed within 450-467 us,
-// with the matrix cores ~28 % busy.
-constexpr int GM_TM = 128;                      // tokens per tile
-constexpr int GM_TN = 256;                      // weight rows per tile
-constexpr int GM_ROWB = BLOCK + 8;              // bytes per LDS row: 32 E4M3 + padding
-constexpr int GM_STAGE = (GM_TM + GM_TN) * GM_ROWB + GM_TM + GM_TN;   // rows, then one scale byte per row
+// One 512-thread workgroup = a tile of TM tokens x TN rows of one matrix; wave (wm, wn),
+// wm < 2, wn < 4, owns MI x NJ fragments of 16 x 16.  K runs in stages of KB 32-element
+// blocks.  A thread converts what it staged to bf16 (scale folded in: exact) as it
+// writes it to LDS, so an element is converted once per workgroup: converted by each
+// wave that reads it (four waves read a row of A, two a row of B) the scaled
+// converters, a quarter of the VALU rate, were the bound.  KB blocks of a row are read by
+// consecutive lanes: 64 or 128 contiguous bytes a request, where one block at a time
+// asked L2 for every line four times.  LDS rows are 16 bytes longer than their blocks,
+// so the 16 rows of a fragment fall on distinct banks.  Two LDS stages, GM_RING stages
+// of bytes in registers; the barriers order LDS only, so those loads stay in flight
+// across them, and loads and stores are unconditional (past K: the last block again,
+// not used), so that no branch makes the compiler wait for them.  Rows past M and N read
+// row 0 (masked at the store).  The products of an output are added block by
+// block in the order of K whatever the tile: all tiles give the same bits.
+// Measured (whole expert, D = 4096, F = 2880, M = 301 / 1000 / 4096): 168 / 177 / 446 us
+// with 128 x 256 tiles of E4M3 in LDS, one block per stage and full fences; now
+// 68 / 130 / 408 us.  128 x 256 tiles with two blocks per stage 146 / 153 / 401 (one
+// workgroup per CU), 64 x 256 tiles 106 / 166 / 552.
+
+// MI x NJ fragments per wave, 2 x 4 waves: a tile of 32 MI tokens x 64 NJ weight rows.
+template <int MI, int NJ, int KB>
+struct GmTile {
+  static constexpr int TM = 32 * MI, TN = 64 * NJ;
+  static constexpr int ROWB = 2 * KB * BLOCK + 16;   // bytes per LDS row: bf16 + padding
+  static constexpr int STAGE = (TM + TN) * ROWB;
+};
 
 constexpr int GM_THREADS = 512;
-#ifndef CACHALOT_GM_RING
-#define CACHALOT_GM_RING 2
-#endif
-constexpr int GM_RING = CACHALOT_GM_RING;       // blocks of bytes in registers
+constexpr int GM_RING = 2;          // stages of bytes in registers
+template <int MI, int NJ, int KB>
 __global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void gemm_kernel(LinearArgs p) {
+  using Tl = GmTile<MI, NJ, KB>;
+  constexpr int GM_TM = Tl::TM, GM_TN = Tl::TN;
+  // staging passes of a stage: 8 bytes of an A row, 16 of a B row per thread and pass
+  constexpr int PA = (KB * GM_TM * 4 + GM_THREADS - 1) / GM_THREADS, PB = (KB * GM_TN * 2 + GM_THREADS - 1) / GM_THREADS;
   extern __shared__ __attribute__((aligned(16))) uint8_t glds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -277,105 +288,144 @@ __global__ __launch_bounds__(GM_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
   const uint8_t* w = mat ? p.w[1] : p.w[0];
   const uint8_t* ws = mat ? p.ws[1] : p.ws[0];
 
-  // staged by this thread: 8 bytes of A row (tid / 4) at byte 8 (tid % 4) of the
-  // block, and 16 bytes of B row (tid / 2) at byte 16 (tid % 2)
-  const int ar = tid >> 2, ah = tid & 3, br = tid >> 1, bh = tid & 1;
-  const int at = t0 + ar, bn = n0 + br;
-  const uint8_t* arow = p.a + (size_t)(at < p.M ? at : 0) * K + 8 * ah;
-  const uint8_t* asc = p.ae + (size_t)(at < p.M ? at : 0) * nkb;
-  const uint8_t* brow = w + (size_t)(bn < p.N ? bn : 0) * K + 16 * bh;
-  const uint8_t* bsc = ws + (size_t)((bn < p.N ? bn : 0) / 32) * nkb;
+  // Staged by this thread: 8 bytes of PA rows of A and 16 of PB rows of B, a row's KB
+  // blocks by consecutive lanes (threads past a smaller tile's rows stage the first
+  // ones again, the same bytes)
+  const int ac = tid % (4 * KB), bc = tid % (2 * KB);   // piece of the row: block ac / 4, bc / 2
+  const uint8_t *arow[PA], *asc[PA], *brow[PB], *bsc[PB];
+  int aoff[PA], boff[PB];                               // where in a stage
+#pragma unroll
+  for (int i = 0; i < PA; ++i) {
+    const int r = (tid + i * GM_THREADS) / (4 * KB) % GM_TM, t = t0 + r < p.M ? t0 + r : 0;
+    arow[i] = p.a + (size_t)t * K + 8 * (ac % 4);
+    asc[i] = p.ae + (size_t)t * nkb;
+    aoff[i] = r * Tl::ROWB + 16 * ac;
+  }
+#pragma unroll
+  for (int i = 0; i < PB; ++i) {
+    const int r = (tid + i * GM_THREADS) / (2 * KB) % GM_TN, n = n0 + r < p.N ? n0 + r : 0;
+    brow[i] = w + (size_t)n * K + 16 * (bc % 2);
+    bsc[i] = ws + (size_t)(n / 32) * nkb;
+    boff[i] = (GM_TM + r) * Tl::ROWB + 32 * bc;
+  }
   struct Raw {
-    uint2 a;
-    uint4 b;
-    uint32_t sa, sb;
+    uint2 a[PA];
+    uint4 b[PB];
+    uint32_t sa[PA], sb[PB];
   };
-  // blocks past K re-read the last one (unconditional loads; never stored)
-  auto load = [&](int kb, Raw& r) {
-    const int k = BLOCK * min(kb, nkb - 1);
-    r.a = *reinterpret_cast<const uint2*>(arow + k);
-    r.b = *reinterpret_cast<const uint4*>(brow + k);
-    r.sa = asc[k / BLOCK];
-    r.sb = bsc[k / BLOCK];
+  // blocks past K re-read the last one (unconditional loads; never used)
+  auto load = [&](int st, Raw& r) {
+    const int ka = min(st * KB + ac / 4, nkb - 1), kb = min(st * KB + bc / 2, nkb - 1);
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      r.a[i] = *reinterpret_cast<const uint2*>(arow[i] + ka * BLOCK);
+      r.sa[i] = asc[i][ka];
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      r.b[i] = *reinterpret_cast<const uint4*>(brow[i] + kb * BLOCK);
+      r.sb[i] = bsc[i][kb];
+    }
   };
   auto store = [&](const Raw& r, uint8_t* buf) {
-    *reinterpret_cast<uint2*>(buf + ar * GM_ROWB + 8 * ah) = r.a;
-    uint2* db = reinterpret_cast<uint2*>(buf + (GM_TM + br) * GM_ROWB + 16 * bh);
-    db[0] = make_uint2(r.b.x, r.b.y);
-    db[1] = make_uint2(r.b.z, r.b.w);
-    uint8_t* sc = buf + (GM_TM + GM_TN) * GM_ROWB;
-    if (ah == 0) sc[ar] = (uint8_t)r.sa;
-    if (bh == 0) sc[GM_TM + br] = (uint8_t)r.sb;
+#pragma unroll
+    for (int i = 0; i < PA; ++i)
+      *reinterpret_cast<bf16x8_t*>(buf + aoff[i]) = to_bf16x8(r.a[i].x, r.a[i].y, e8m0_to_f32(r.sa[i]));
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const float eb = e8m0_to_f32(r.sb[i]);
+      bf16x8_t* db = reinterpret_cast<bf16x8_t*>(buf + boff[i]);
+      db[0] = to_bf16x8(r.b[i].x, r.b[i].y, eb);
+      db[1] = to_bf16x8(r.b[i].z, r.b[i].w, eb);
+    }
   };
   // the 8 values of lane (fr, fg) of a fragment whose 16 rows start at LDS row `row0`
   auto frag = [&](const uint8_t* buf, int row, int fg) {
-    const uint2 v = *reinterpret_cast<const uint2*>(buf + row * GM_ROWB + 8 * fg);
-    const uint32_t sc = buf[(GM_TM + GM_TN) * GM_ROWB + row];
-    return to_bf16x8(v.x, v.y, e8m0_to_f32(sc));
+    return *reinterpret_cast<const bf16x8_t*>(buf + row * Tl::ROWB + 16 * fg);
   };
 
-  f32x4_t acc[4][4];
+  f32x4_t acc[MI][NJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   const int fr = lane & 15, fg = lane >> 4;   // fragment row / column and k group
-  // a ring of GM_RING blocks in registers, two in LDS; GM_RING blocks per trip so the
+  // a ring of GM_RING stages in registers, two in LDS; GM_RING stages per trip so the
   // ring index is a constant
+  const int nst = (nkb + KB - 1) / KB;
   Raw ring[GM_RING];
 #pragma unroll
   for (int r = 0; r < GM_RING; ++r) load(r, ring[r]);
   store(ring[0], glds);
-  __syncthreads();
-  for (int kb0 = 0; kb0 < nkb; kb0 += GM_RING) {
+  lds_sync();
+  for (int st0 = 0; st0 < nst; st0 += GM_RING) {
 #pragma unroll
     for (int u = 0; u < GM_RING; ++u) {
-      const int kb = kb0 + u;
-      if (kb < nkb) {
-        const uint8_t* buf = glds + (kb & 1) * GM_STAGE;
-        load(kb + GM_RING, ring[u]);   // the slot of block kb, already in LDS
-        bf16x8_t af[4];
+      const int st = st0 + u;
+      load(st + GM_RING, ring[u]);   // the slot of stage st, already in LDS
 #pragma unroll
-        for (int i = 0; i < 4; ++i) af[i] = frag(buf, 64 * wm + 16 * i + fr, fg);
+      for (int b = 0; b < KB; ++b) {
+        if (st * KB + b >= nkb) break;
+        const uint8_t* buf = glds + (st & 1) * Tl::STAGE + 2 * BLOCK * b;
+        bf16x8_t af[MI];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const bf16x8_t bfr = frag(buf, GM_TM + 64 * wn + 16 * j + fr, fg);
+        for (int i = 0; i < MI; ++i) af[i] = frag(buf, 16 * MI * wm + 16 * i + fr, fg);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i][j] = mfma_bf16(af[i], bfr, acc[i][j]);
+        for (int j = 0; j < NJ; ++j) {
+          const bf16x8_t bfr = frag(buf, GM_TM + 16 * NJ * wn + 16 * j + fr, fg);
+#pragma unroll
+          for (int i = 0; i < MI; ++i) acc[i][j] = mfma_bf16(af[i], bfr, acc[i][j]);
         }
-        if (kb + 1 < nkb) store(ring[(u + 1) % GM_RING], glds + ((kb + 1) & 1) * GM_STAGE);
-        __syncthreads();
       }
+      store(ring[(u + 1) % GM_RING], glds + ((st + 1) & 1) * Tl::STAGE);
+      lds_sync();
     }
   }
   // D[r][c] of a 16 x 16 tile: lane c + 16 (r / 4), register r % 4
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int n = n0 + 64 * wn + 16 * j + fr;
+  for (int j = 0; j < NJ; ++j) {
+    const int n = n0 + 16 * NJ * wn + 16 * j + fr;
     if (n >= p.N) continue;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int t = t0 + 64 * wm + 16 * i + 4 * fg + v;
+        const int t = t0 + 16 * MI * wm + 16 * i + 4 * fg + v;
         if (t < p.M) p.out[(size_t)t * p.ldo + mat * p.N + n] = f32_to_bf16(acc[i][j][v]);
       }
   }
 }
 
+template <int MI, int NJ, int KB>
+int launch_gemm(const LinearArgs& a, int nmat, hipStream_t s) {
+  using Tl = GmTile<MI, NJ, KB>;
+  const dim3 grid((unsigned)(nmat * ((a.N + Tl::TN - 1) / Tl::TN)), (unsigned)((a.M + Tl::TM - 1) / Tl::TM));
+  auto k = gemm_kernel<MI, NJ, KB>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          2 * Tl::STAGE) != hipSuccess)
+    return fail(CACHALOT_EHIP, "fp8 linear: cannot grant %d bytes of LDS", 2 * Tl::STAGE);
+  hipLaunchKernelGGL(k, grid, dim3(GM_THREADS), 2 * Tl::STAGE, s, a);
+  return check_launch("fp8 gemm");
+}
+
 // Tile choice: token-tiled GEMV (one 16-token tile per workgroup, 8 chunks of
-// every wave in flight) for decode-sized M; 128 x 128 LDS tiles for many tokens.
+// every wave in flight) for decode-sized M (M = 64: 46 us against 50 us for the GEMM
+// of smallest tiles at M = 65); above, the smallest of the LDS tiles that gives each of
+// the 256 CUs at most one workgroup: up to there a smaller tile only shortens what each
+// workgroup does, past it a second round costs more than it.  Whole expert in us,
+// 32 x 64 / 64 x 128 / 128 x 128 tiles throughout: D = 5120, F = 2304, M = 65 (216 and
+// 240 workgroups of 32 x 64) 42 / 67 / 93, M = 301 (180 and 200 of 64 x 128) 94 / 71 / 98,
+// M = 512 (288 and 320) 131 / 108 / 99; D = 4096, F = 2880, M = 128 (360 and 256 of
+// 32 x 64) 52 / 65 / 90, M = 768 (552 and 384 of 64 x 128) 183 / 135 / 128.
 int launch_linear(const LinearArgs& a, int nmat, hipStream_t s) {
   if (a.M > 64) {
-    const dim3 grid((unsigned)(nmat * ((a.N + GM_TN - 1) / GM_TN)), (unsigned)((a.M + GM_TM - 1) / GM_TM));
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            2 * GM_STAGE) != hipSuccess)
-      return fail(CACHALOT_EHIP, "fp8 linear: cannot grant %d bytes of LDS", 2 * GM_STAGE);
-    hipLaunchKernelGGL(gemm_kernel, grid, dim3(GM_THREADS), 2 * GM_STAGE, s, a);
-  } else {
-    const dim3 grid((unsigned)(nmat * a.N / 16), (unsigned)((a.M + 15) / 16));
-    hipLaunchKernelGGL((linear_kernel<1, 1, 8>), grid, dim3(256), 0, s, a);
+    auto fits = [&](long tm, long tn) { return nmat * ((a.N + tn - 1) / tn) * ((a.M + tm - 1) / tm) <= 256; };
+    if (fits(32, 64)) return launch_gemm<1, 1, 4>(a, nmat, s);
+    if (fits(64, 128)) return launch_gemm<2, 2, 2>(a, nmat, s);
+    return launch_gemm<4, 2, 2>(a, nmat, s);
   }
+  const dim3 grid((unsigned)(nmat * a.N / 16), (unsigned)((a.M + 15) / 16));
+  hipLaunchKernelGGL((linear_kernel<1, 1, 8>), grid, dim3(256), 0, s, a);
   return check_launch("fp8 linear");
 }
 

@@ -100,6 +100,26 @@ def _one_ulp_of_exact(got, q, e, w, s):
     return np.all(np.abs(got - exact) <= bf16_ulp(exact) + 2.0 ** -20 * mag)
 
 
+@pytest.mark.parametrize("m,k,n", [(65, 32, 64), (97, 160, 96), (1025, 96, 544), (1100, 352, 512), (2100, 96, 1120),
+                                   (2049, 224, 1088)])
+def test_fp8_linear_tiles_agree(cuda, m, k, n):
+    """Each LDS tile of the many-token GEMM (32 x 64, 64 x 128, 128 x 128), ragged in tokens, rows and blocks per
+    stage: the rows of a call in the smallest tile bit for bit (the products are added in one order), and those
+    within the linear's bar."""
+    from cachalot_amd.shared_expert import fp8_linear
+
+    rng = np.random.default_rng(SEED + m + k)
+    w, s = _weights(rng, n, k)
+    x = round_bf16(rng.standard_normal((m, k)).astype(np.float32))
+    xd, wd, sd = _to_dev_bf16(x, cuda), _dev(w, cuda), _dev(s, cuda)
+    got = fp8_linear(xd, wd, sd)
+    rows = [0, 31, 32, 63, 64, m // 2, m - 65, m - 1]
+    small = torch.cat([fp8_linear(xd[r0:r0 + 65], wd, sd) for r0 in range(0, m - 64, 65)])
+    assert torch.equal(got[:small.shape[0]].view(torch.int16), small.view(torch.int16))
+    q, e = ofp8.act_quant(x[rows])
+    assert _one_ulp_of_exact(_bf16_np(got)[rows], q, e, w, s), (m, k, n)
+
+
 @pytest.mark.parametrize("m,d,f", [(1, 4096, 2880), (1, 5120, 2304), (3, 4096, 2880), (4, 1024, 2304),
                                    (5, 256, 192), (130, 1024, 640), (200, 4096, 2880)])
 def test_shared_expert_matches_oracle(cuda, m, d, f):
