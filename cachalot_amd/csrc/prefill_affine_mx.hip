@@ -233,7 +233,8 @@ __global__ void __launch_bounds__(P3_THREADS) p4_kernel(MxArgs g, int slices) {
         // this wave's loads of chunk c have landed (the last code load is consumed here;
         // the scale group, issued before it, first), then every wave's; the first barrier
         // also publishes the staged sums
-        asm volatile("" ::"v"(ring[u % 2].codes[NP - 1][1].w) : "memory");
+        const uint4& lastc = ring[u % 2].codes[NP - 1][1];
+        asm volatile("" ::"v"(ak_bits(AK) == 2 ? lastc.y : lastc.w) : "memory");
         lds_sync();
         if ((u + 1) % 4 == 0) load_sg(min((c + 1) / 4, nq - 1), sg[((u + 1) / 4) % 2]);
         p4_issue<AK, NM, NF>(abuf + ((u + 1) % 2) * P3_ABYTES, asrc, base, woff, nrow, min(c + 1, nch - 1), kh, wave,
