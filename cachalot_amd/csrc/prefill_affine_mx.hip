@@ -12,12 +12,18 @@ using namespace pmx;
 // 16 x 16 x 128 instruction holds two such groups).  Reference semantics as
 // prefill_mx.hip (expert_affine.py:84-99, the group formula of minimax/codes_qmv.py:86-100).
 //
+// VALU bound: the fold (256 fma per chunk and wave, as long as the instructions
+// themselves) and the spread of the codes.  One 3-bit g64 layer over 2048 tokens,
+// D = 5120, F = 2304: 3397 us with 3-bit codes as fp8 bytes, 2954 us as fp6 fields.
+//
 // Built with -mllvm -amdgpu-mfma-vgpr-form=true: the tiles stay in VGPRs, where the
 // per-group fold reads them (with AGPR tiles every fold read is a copy).
 //
 // Operand layout (fp8, measured): lane l holds row (A) or column (B) l & 31; its
 // registers 0..3 carry elements 16 (l >> 5) .. + 15 of the 64, registers 4..7 elements 32 + 16 (l >> 5) .. + 15; the scale of block b
-// (elements 32 b .. 32 b + 31) of row r comes from lane 32 b + r.  Result register j of
+// (elements 32 b .. 32 b + 31) of row r comes from lane 32 b + r.  An fp6 column (3-bit
+// codes): elements 32 (l >> 5) .. + 31 in order, six registers; the planes of 3-bit banks
+// hold each block's even elements, then its odd ones (plane_pos).  Result register j of
 // lane l: row 8 (j / 4) + 4 (l >> 5) + (j & 3), column l & 31.
 //
 // One 256-thread workgroup = the 64-row M tile x 32 NF weight rows per wave of each of
@@ -25,17 +31,31 @@ using namespace pmx;
 // mapping and the plane writers are those of p3_kernel.
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 constexpr int P4_TB = P3_MT / 32;   // 32-row token blocks
+constexpr uint32_t E8M0_2P3 = 0x01010101u * 130;
+
+// The fp6 B operand of a lane from its 32 3-bit codes (12 bytes): code q is the field q,
+// E2M3 q / 8 (B scale 2^3).  Every second code already lies alone in a 6-bit field, so
+// the even codes are three masks, the odd ones the same three bits on: nine instructions,
+// where one byte per code took some sixty and bounded the kernel.
+__device__ __forceinline__ i32x8_t aff3_code_fields(const uint4& w) {
+  constexpr uint32_t M0 = 0xC71C71C7u, M1 = 0x71C71C71u, M2 = 0x1C71C71Cu;
+  const uint32_t o1 = __builtin_amdgcn_alignbit(w.y, w.x, 3), o2 = __builtin_amdgcn_alignbit(w.z, w.y, 3);
+  return i32x8_t{(int)(w.x & M0), (int)(w.y & M1), (int)(w.z & M2), (int)(o1 & M0), (int)(o2 & M1),
+                 (int)((w.z >> 3) & M2), 0, 0};
+}
 
 // The tile stays in VGPRs (the fold reads it there); ZERO: the accumulator input is the
 // inline constant 0.
-template <int OPSEL_A, bool ZERO>
+template <int BITS, int OPSEL_A, bool ZERO>
 __device__ __forceinline__ f32x16_t mfma32_plane(const i32x8_t& a, const i32x8_t& b, f32x16_t c, uint32_t sa) {
+  constexpr int FMT_B = BITS == 3 ? 2 : 0;                          // fp6 E2M3 or fp8 E4M3
+  constexpr uint32_t SCALE_B = BITS == 3 ? E8M0_2P3 : E8M0_2P9;
   f32x16_t d;
   if constexpr (ZERO) {
     const f32x16_t z = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    d = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, z, 0, 0, OPSEL_A, (int)sa, 0, (int)E8M0_2P9);
+    d = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, z, 0, FMT_B, OPSEL_A, (int)sa, 0, (int)SCALE_B);
   } else {
-    d = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, OPSEL_A, (int)sa, 0, (int)E8M0_2P9);
+    d = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, FMT_B, OPSEL_A, (int)sa, 0, (int)SCALE_B);
   }
   return d;
 }
@@ -45,7 +65,8 @@ struct P4Chunk {
   uint4 codes[NP][2];   // per (matrix, weight block) pair and half of the chunk: the lane's two runs
 };
 
-// Codes of half h of chunk c for lane half kh: runs at elements 64 h + 16 kh and + 32,
+// Codes of half h of chunk c for lane half kh: 3-bit, the 12 bytes of the 32 elements
+// from 64 h + 32 kh; 2- and 4-bit, runs at elements 64 h + 16 kh and + 32,
 // 2 BITS bytes each, loaded as whole words as in p3_issue_aff.  (The scales and biases
 // come in groups of eight, p4_kernel.)
 template <int AK, int NM, int NF>
@@ -64,6 +85,11 @@ __device__ __forceinline__ void p4_issue(uint8_t* stage, const uint8_t* (&asrc)[
       const uint8_t* row = base + woff[m] + nrow[f] * row_bytes;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
+        if constexpr (BITS == 3) {
+          const uint3 v = *reinterpret_cast<const uint3*>(row + min(c * CB + 24 * h + 12 * kh, row_bytes - 12));
+          out.codes[m * NF + f][h] = make_uint4(v.x, v.y, v.z, 0u);
+          continue;
+        }
         const int r0 = (2 * BITS * (4 * h + kh)) & ~3, r1 = (2 * BITS * (4 * h + kh) + 4 * BITS) & ~3;
         const int o0 = min(c * CB + r0, row_bytes - LB), o1 = min(c * CB + r1, row_bytes - LB);
         if constexpr (BITS == 2) {
@@ -96,7 +122,8 @@ __device__ __forceinline__ void p4_compute(const uint8_t* ab, const uint8_t* sbu
     for (int h = 0; h < 2; ++h) {
       sc[p][h] = scale_bits_to_f32((uint16_t)(sw[p] >> (16 * h)), f16);
       bi[p][h] = scale_bits_to_f32((uint16_t)(bw[p] >> (16 * h)), f16);
-      b[p][h] = aff_code_bytes<ak_bits(AK)>(ch.codes[p][h], kh);
+      if constexpr (ak_bits(AK) == 3) b[p][h] = aff3_code_fields(ch.codes[p][h]);
+      else b[p][h] = aff_code_bytes<ak_bits(AK)>(ch.codes[p][h], kh);
     }
 #pragma unroll
   for (int tb = 0; tb < P4_TB; ++tb) {
@@ -116,9 +143,9 @@ __device__ __forceinline__ void p4_compute(const uint8_t* ab, const uint8_t* sbu
       const i32x8_t alo = {(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
       f32x16_t d[NP];
 #pragma unroll
-      for (int p = 0; p < NP; ++p) d[p] = mfma32_plane<0, true>(ahi, b[p][h], d[p], sa);
+      for (int p = 0; p < NP; ++p) d[p] = mfma32_plane<ak_bits(AK), 0, true>(ahi, b[p][h], d[p], sa);
 #pragma unroll
-      for (int p = 0; p < NP; ++p) d[p] = mfma32_plane<1, false>(alo, b[p][h], d[p], sa);
+      for (int p = 0; p < NP; ++p) d[p] = mfma32_plane<ak_bits(AK), 1, false>(alo, b[p][h], d[p], sa);
       float sx[16];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -234,7 +261,7 @@ __global__ void __launch_bounds__(P3_THREADS) p4_kernel(MxArgs g, int slices) {
         // the scale group, issued before it, first), then every wave's; the first barrier
         // also publishes the staged sums
         const uint4& lastc = ring[u % 2].codes[NP - 1][1];
-        asm volatile("" ::"v"(ak_bits(AK) == 2 ? lastc.y : lastc.w) : "memory");
+        asm volatile("" ::"v"(ak_bits(AK) == 2 ? lastc.y : ak_bits(AK) == 3 ? lastc.z : lastc.w) : "memory");
         lds_sync();
         if ((u + 1) % 4 == 0) load_sg(min((c + 1) / 4, nq - 1), sg[((u + 1) / 4) % 2]);
         p4_issue<AK, NM, NF>(abuf + ((u + 1) % 2) * P3_ABYTES, asrc, base, woff, nrow, min(c + 1, nch - 1), kh, wave,
@@ -281,7 +308,8 @@ __global__ void __launch_bounds__(P3_THREADS) p4_kernel(MxArgs g, int slices) {
         const float s = hv * __uint_as_float((uint32_t)(127 - E) << 23);
         const uint32_t hi = mx::f32_to_e4m3(s);
         const uint32_t lo = mx::f32_to_e4m3((s - mx::e4m3_to_f32(hi)) * 16.0f);
-        uint8_t* p = g.hp + ((size_t)prow * g.hkch + (n >> 7)) * P3_ROWB + (n & 127);
+        uint8_t* p = g.hp + ((size_t)prow * g.hkch + (n >> 7)) * P3_ROWB + (n & 96) +
+                     plane_pos<p4_order(AK)>(n & 31);
         p[0] = (uint8_t)hi;
         p[128] = (uint8_t)lo;
         float hs = row16_sum(hv);

@@ -71,7 +71,9 @@ __host__ __device__ inline int scale_row_bytes(int K) { return (K / 32 * 2 + 15)
 // Position along K of element n of a 32-element block in the planes of the few-row
 // kernels (small_rows_mx.hip), the order its BITS-bit codes spread to fp4 in: 2-bit even
 // elements of each 16, then odd; 3-bit code 4t + r at 3t + r (r < 3), codes 4t + 3 in the
-// last eight; others natural.
+// last eight; others natural.  PLANE_EVEN_ODD: the even elements, then the odd ones (3-bit
+// groups of 64 in prefill_affine_mx.hip, whose codes spread to fp6 in that order).
+constexpr int PLANE_EVEN_ODD = 32;
 template <int BITS>
 __host__ __device__ inline int plane_pos(int n) {
   if (BITS == 2) return (n & 16) + ((n & 1) ? 8 + ((n & 15) >> 1) : (n & 15) >> 1);
@@ -79,7 +81,13 @@ __host__ __device__ inline int plane_pos(int n) {
     const int t = n >> 2, r = n & 3;
     return r < 3 ? 3 * t + r : 24 + ((0x65274130 >> (4 * t)) & 15);
   }
+  if (BITS == PLANE_EVEN_ODD) return (n & 1) * 16 + (n >> 1);
   return n;
+}
+
+// The order the planes of a kind's 64-row-tile kernels are in.
+constexpr int p4_order(int ak) {
+  return ak_bytes(ak) && ak_bits(ak) == 3 && ak_group(ak) == 64 ? PLANE_EVEN_ODD : 0;
 }
 
 // Place of 32-element block b of a 128-element chunk in those planes (its own inverse):

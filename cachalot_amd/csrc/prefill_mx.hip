@@ -175,6 +175,12 @@ __global__ void __launch_bounds__(256) x_planes_rows_kernel(const uint16_t* __re
     *reinterpret_cast<uint32_t*>(dst + 8) = __builtin_amdgcn_perm(hi.y, hi.x, 0x07050301u);
     *reinterpret_cast<uint32_t*>(dst + 128) = __builtin_amdgcn_perm(lo.y, lo.x, 0x06040200u);
     *reinterpret_cast<uint32_t*>(dst + 136) = __builtin_amdgcn_perm(lo.y, lo.x, 0x07050301u);
+  } else if constexpr (BITS == PLANE_EVEN_ODD) {
+    uint8_t* dst = chunk + (col & 96) + (g8 & 3) * 4;
+    *reinterpret_cast<uint32_t*>(dst) = __builtin_amdgcn_perm(hi.y, hi.x, 0x06040200u);
+    *reinterpret_cast<uint32_t*>(dst + 16) = __builtin_amdgcn_perm(hi.y, hi.x, 0x07050301u);
+    *reinterpret_cast<uint32_t*>(dst + 128) = __builtin_amdgcn_perm(lo.y, lo.x, 0x06040200u);
+    *reinterpret_cast<uint32_t*>(dst + 144) = __builtin_amdgcn_perm(lo.y, lo.x, 0x07050301u);
   } else {
     uint8_t* dst = chunk + (col & 96);
     const uint32_t hw[2] = {hi.x, hi.y}, lw[2] = {lo.x, lo.y};
@@ -784,7 +790,7 @@ int launch_p3(const uint16_t* x, int T, const uint8_t* pool, const decode::Layou
                                      F, k, limit, ws, y);
   constexpr bool Q2 = ak_fold(AK);
   constexpr int GPC = ak_gpc(AK);
-  int rc = launch_x_planes_rows<0>(c, x, T, D, Q2 ? 128 / GPC : 0, s);
+  int rc = launch_x_planes_rows<p4_order(AK)>(c, x, T, D, Q2 ? 128 / GPC : 0, s);
   if (rc) return rc;
   const MxArgs &gu = c.gu, &dn = c.dn;
   const int sbx = c.sbx, sbh = c.sbh, fch = c.fch;
