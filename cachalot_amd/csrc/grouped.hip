@@ -1069,8 +1069,8 @@ inline bool prefill_bf16_requested() {
 // experts top-6, against the path on the other side of the line, us:
 //   FP4: 200 tokens (3.1 per expert) 1366 against 1745 (bf16-MFMA 16-row tiles), 400
 //     (6.3) 1884 against 1752 (64-row tiles): up to 5;
-//   3-bit g64: 200 tokens 1940 against 5926 (bf16-MFMA), 256 2400 against 2650 (64-row), 400
-//     3300 against 2720: up to 4, the same for the other widths and groups;
+//   3-bit g64: 200 tokens 1940 against 5926 (bf16-MFMA), 256 2400 against 2190 (64-row, once
+//     its codes went in as fp6; 2650 before), 400 3300 against 2720 (before): up to 4, the same for the other widths and groups;
 //   2-bit g128: 64 tokens (1 per expert) 573 against 535 (one-token items per row), 128 (2)
 //     848 against 918, 400 1440 against 1703 (64-row), 600 (9.4) 2050 against 1850: 1.5 to 8.
 inline bool small_rows_wanted(int kind, int rows, int E) {

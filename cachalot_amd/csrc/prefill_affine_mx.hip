@@ -14,7 +14,7 @@ using namespace pmx;
 //
 // VALU bound: the fold (256 fma per chunk and wave, as long as the instructions
 // themselves) and the spread of the codes.  One 3-bit g64 layer over 2048 tokens,
-// D = 5120, F = 2304: 3397 us with 3-bit codes as fp8 bytes, 2954 us as fp6 fields.
+// D = 4096, F = 2880: 3397 us with 3-bit codes as fp8 bytes, 2954 us as fp6 fields.
 //
 // Built with -mllvm -amdgpu-mfma-vgpr-form=true: the tiles stay in VGPRs, where the
 // per-group fold reads them (with AGPR tiles every fold read is a copy).

@@ -23,7 +23,7 @@
 //           then lo bytes 128..255, element order;
 //   scales  [rows][sb B]: per 32-element block b, bytes 2b (hi) and 2b + 1 (lo),
 //           sb a multiple of 16.
-// x_planes_kernel writes x's planes per token; the gate/up kernel's epilogue
+// x_planes_rows_kernel writes x's planes per token; the gate/up kernel's epilogue
 // writes h's planes per permuted row (columns past F are zero, so K_pad = F
 // rounded up to 128 reads zeros there).
 //
