@@ -36,10 +36,10 @@ CFLAGS = [
 ]
 
 
-# Per-file flags.  prefill_affine_mx.hip, small_rows_mx.hip: matrix-core results in VGPRs,
+# Per-file flags.  prefill_affine_mx.hip, small_rows.hip: matrix-core results in VGPRs,
 # where their per-group folds read them (the other kernels keep their accumulators in AGPRs).
 _VGPR_TILES = ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]
-FILE_FLAGS = {"prefill_affine_mx.hip": _VGPR_TILES, "small_rows_mx.hip": _VGPR_TILES}
+FILE_FLAGS = {"prefill_affine_mx.hip": _VGPR_TILES, "small_rows.hip": _VGPR_TILES}
 
 
 def sources() -> list[Path]:

@@ -70,15 +70,13 @@ int launch_prefill_mx(const uint16_t* x, int T, const uint8_t* pool, const decod
                       int max_tiles, const int32_t* row_token, const int32_t* row_slot, const float* row_w, int D,
                       int F, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s);
 bool prefill_mx_q2_supported(int D, int F, const decode::Layout& L);
-// few rows per expert on the block-scaled matrix cores (small_rows_mx.hip, prefill_mx.hip);
-// bits 0: FP4
-int small_rows_mt(int ak);
-int small_rows_ak(int bits, int group);
-bool small_rows_supported(int ak, int D, int F, const decode::Layout& L);
-int launch_prefill_small(int bits, int group, const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
-                         const int4* recs, const int32_t* recs_n, const int32_t* row_token,
-                         const int32_t* row_slot, const float* row_w, int D, int F, int k, float limit, uint8_t* ws,
-                         uint16_t* y, hipStream_t s);
+// few rows per expert (small_rows.hip); bits 0: FP4
+int small_rows_mt(int bits, int group);
+bool small_rows_supported(int bits, int group, int D, int F, const decode::Layout& L);
+size_t small_rows_ws_bytes(int T, int k, int D, int F);
+int launch_small_rows(int bits, int group, const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
+                      const int4* recs, const int32_t* recs_n, const int32_t* row_token, const int32_t* row_slot,
+                      const float* row_w, int D, int F, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s);
 int launch_prefill_mx_q2(const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
                          const int32_t* slot_table, const int32_t* offsets, const int2* tiles,
                          const int32_t* tiles_n, int max_tiles, const int32_t* row_token, const int32_t* row_slot,
@@ -1023,7 +1021,7 @@ inline GroupedWs grouped_ws(int T, int k, int E, int D, int F) {
   const size_t hid = std::max((size_t)rows * F * sizeof(uint16_t), (size_t)rows * ((F + 127) / 128) * 320);
   w.xplanes = w.hidden + align256(hid);
   w.mx = w.xplanes + align256((size_t)T * ((D + 127) / 128) * 320);
-  w.total = w.mx + (k > 0 && D > 0 ? prefill_mx_ws_bytes(T, k, D, F) : 0);
+  w.total = w.mx + (k > 0 && D > 0 ? std::max(prefill_mx_ws_bytes(T, k, D, F), small_rows_ws_bytes(T, k, D, F)) : 0);
   return w;
 }
 
@@ -1063,7 +1061,7 @@ inline bool prefill_bf16_requested() {
   return env && env[0] == '1';
 }
 
-// Where the few-row weight stream (small_rows_mx.hip) is the faster one, in routes per
+// Where the few-row weight stream (small_rows.hip) is the faster one, in routes per
 // expert.  It reads an expert's weights once per 8 (4) rows, the 64-row tiles once per 64
 // but at a lower rate while tiles are nearly empty.  Per layer at D 4096 x F 2880, 384
 // experts top-6, against the path on the other side of the line, us:
@@ -1114,11 +1112,10 @@ int launch_grouped(const uint16_t* x, const uint8_t* pool, const cachalot_expert
   // tiles of 64 rows when experts see many tokens, 16 for batched decode
   const int MT = T * k >= 4 * E ? 64 : 16;
   uint32_t* zeros = reinterpret_cast<uint32_t*>(ws + wo.tiles_n + 128);
-  // few rows per expert: the weight stream of small_rows_mx.hip
+  // few rows per expert: the weight stream of small_rows.hip
   constexpr int SBITS = KIND == KIND_FP4 ? 0 : KIND == KIND_Q2 ? 2 : aff_bits(KIND);
   constexpr int SGROUP = is_aff(KIND) ? aff_group(KIND) : KC;
-  const int sak = small_rows_ak(SBITS, SGROUP), smt = small_rows_mt(sak);
-  const bool small = small_rows_wanted(KIND, T * k, E) && small_rows_supported(sak, D, F, L) &&
+  const bool small = small_rows_wanted(KIND, T * k, E) && small_rows_supported(SBITS, SGROUP, D, F, L) &&
                      !small_tiles_requested() && !prefill_bf16_requested();
   const bool batched = KIND == KIND_Q2 && MT == 16 && q2mx_supported(D, F, k) && !small && !small_tiles_requested();
   // routes given: permuted by the batched prep launch when one workgroup holds them, else here
@@ -1140,11 +1137,12 @@ int launch_grouped(const uint16_t* x, const uint8_t* pool, const cachalot_expert
   if (rc) return rc;
   if (small) {
     int4* recs = reinterpret_cast<int4*>(ws + wo.tiles);
-    hipLaunchKernelGGL(tile_recs_kernel, dim3(1), dim3(1024), 0, s, offsets, slot_table, E, smt, recs, tiles_n);
+    hipLaunchKernelGGL(tile_recs_kernel, dim3(1), dim3(1024), 0, s, offsets, slot_table, E,
+                       small_rows_mt(SBITS, SGROUP), recs, tiles_n);
     rc = check_launch("tile_recs_kernel");
     if (rc) return rc;
-    return launch_prefill_small(SBITS, SGROUP, x, T, pool, L, recs, tiles_n, row_token, row_slot, row_w,
-                                D, F, k, limit, ws + wo.mx, y, s);
+    return launch_small_rows(SBITS, SGROUP, x, T, pool, L, recs, tiles_n, row_token, row_slot, row_w, D, F, k, limit,
+                             ws + wo.mx, y, s);
   }
   const int max_tiles = (T * k) / MT + std::min(E, T * k) + 1;
   if (KIND == KIND_FP4 && MT == 64 && prefill_mx_supported(D, F, L) && !small_tiles_requested() &&

@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(P3_THREADS) p4_kernel(MxArgs g, int slices) {
         const uint32_t hi = mx::f32_to_e4m3(s);
         const uint32_t lo = mx::f32_to_e4m3((s - mx::e4m3_to_f32(hi)) * 16.0f);
         uint8_t* p = g.hp + ((size_t)prow * g.hkch + (n >> 7)) * P3_ROWB + (n & 96) +
-                     plane_pos<p4_order(AK)>(n & 31);
+                     plane_pos<ak_even_odd(AK)>(n & 31);
         p[0] = (uint8_t)hi;
         p[128] = (uint8_t)lo;
         float hs = row16_sum(hv);

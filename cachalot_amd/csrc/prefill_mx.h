@@ -27,7 +27,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 // Weight kinds of p3_kernel (AK): FP4; 2-bit g128 with the codes as fp4 operands;
 // (BITS << 8) | G for affine codes as fp8 operands (code q as the E4M3 byte q, which
-// is q * 2^-9 -- subnormal below 8 -- with B scale 2^9).
+// is q * 2^-9 -- subnormal below 8 -- with B scale 2^9), 3-bit groups of 64 as fp6
+// operands (prefill_affine_mx.hip).
 constexpr int AK_FP4 = 0;
 constexpr int AK_Q2 = 1;
 constexpr int ak_aff(int bits, int g) { return (bits << 8) | g; }
@@ -63,39 +64,16 @@ struct MxArgs {
   uint16_t* y;                // down: [T, k, N]
   const float* asum;          // 2-bit: chunk sums of the A source rows [source rows][kch]
   float* hsum;                // 2-bit gate/up: chunk sums of h [rows][hkch]
-  const int4* recs;           // few-row kernels: the tiles as (expert, first row, end row, slot)
 };
 
 __host__ __device__ inline int scale_row_bytes(int K) { return (K / 32 * 2 + 15) / 16 * 16; }
 
-// Position along K of element n of a 32-element block in the planes of the few-row
-// kernels (small_rows_mx.hip), the order its BITS-bit codes spread to fp4 in: 2-bit even
-// elements of each 16, then odd; 3-bit code 4t + r at 3t + r (r < 3), codes 4t + 3 in the
-// last eight; others natural.  PLANE_EVEN_ODD: the even elements, then the odd ones (3-bit
-// groups of 64 in prefill_affine_mx.hip, whose codes spread to fp6 in that order).
-constexpr int PLANE_EVEN_ODD = 32;
-template <int BITS>
-__host__ __device__ inline int plane_pos(int n) {
-  if (BITS == 2) return (n & 16) + ((n & 1) ? 8 + ((n & 15) >> 1) : (n & 15) >> 1);
-  if (BITS == 3) {
-    const int t = n >> 2, r = n & 3;
-    return r < 3 ? 3 * t + r : 24 + ((0x65274130 >> (4 * t)) & 15);
-  }
-  if (BITS == PLANE_EVEN_ODD) return (n & 1) * 16 + (n >> 1);
-  return n;
-}
-
-// The order the planes of a kind's 64-row-tile kernels are in.
-constexpr int p4_order(int ak) {
-  return ak_bytes(ak) && ak_bits(ak) == 3 && ak_group(ak) == 64 ? PLANE_EVEN_ODD : 0;
-}
-
-// Place of 32-element block b of a 128-element chunk in those planes (its own inverse):
-// the 2-bit codes reach the lane groups in the order 0, 2, 1, 3.
-template <int BITS>
-__host__ __device__ inline int block_at(int b) {
-  return BITS == 2 && (b == 1 || b == 2) ? 3 - b : b;
-}
+// Whether the planes of a kind hold each 32-element block's even elements, then its odd
+// ones (3-bit groups of 64 in prefill_affine_mx.hip, whose codes spread to fp6 in that
+// order), and the place of element n of a block.
+constexpr bool ak_even_odd(int ak) { return ak_bytes(ak) && ak_bits(ak) == 3 && ak_group(ak) == 64; }
+template <bool EVEN_ODD>
+__host__ __device__ inline int plane_pos(int n) { return EVEN_ODD ? (n & 1) * 16 + (n >> 1) : n; }
 
 // Plane scale exponent of a block whose largest magnitude is m: E = e(m) - 7,
 // clamped so that both E8M0 bytes (E + 127, E + 123) are finite scales.

@@ -61,9 +61,6 @@
 
 namespace cachalot {
 
-// few rows per expert, every bank kind (small_rows_mx.hip)
-int launch_small_rows(int ak, const pmx::MxArgs& gu, const pmx::MxArgs& dn, hipStream_t s);
-
 // affine groups of 64 (prefill_affine_mx.hip)
 int launch_prefill_affine_g64(int ak, const pmx::MxArgs& gu, int s_gu, size_t lds_gu, const pmx::MxArgs& dn,
                               int s_dn, size_t lds_dn, int tiles8, hipStream_t s);
@@ -124,9 +121,8 @@ __device__ __forceinline__ void encode8(const float (&v)[8], float inv, uint2& h
 }
 
 // x [T, D] bf16 -> planes and scales per token.  One thread = 8 values; the four
-// threads of an aligned lane quad hold one 32-element block.  BITS: the element order
-// inside a block (plane_pos; 0 natural).
-template <int BITS>
+// threads of an aligned lane quad hold one 32-element block.  EVEN_ODD: plane_pos.
+template <bool EVEN_ODD>
 __global__ void __launch_bounds__(256) x_planes_rows_kernel(const uint16_t* __restrict__ x, int T, int D,
                                                             uint8_t* __restrict__ xp, uint8_t* __restrict__ xs,
                                                             int sb, float* __restrict__ xsum, int gsum) {
@@ -152,44 +148,28 @@ __global__ void __launch_bounds__(256) x_planes_rows_kernel(const uint16_t* __re
   uint2 hi, lo;
   encode8(v, __uint_as_float((uint32_t)(127 - E) << 23), hi, lo);
   // the group sums of affine banks' group formula (gsum = 128: 16 threads per group,
-  // 64: 8 threads, 32: 4 threads)
+  // 64: 8 threads)
   float cs = 0.0f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) cs = cs + v[j];
   cs = cs + __uint_as_float(xor1_u32(__float_as_uint(cs)));
   cs = cs + __uint_as_float(xor2_u32(__float_as_uint(cs)));
-  if (gsum >= 64) cs = cs + __uint_as_float(mirror8_u32(__float_as_uint(cs)));
+  cs = cs + __uint_as_float(mirror8_u32(__float_as_uint(cs)));
   if (gsum == 128) cs = cs + __uint_as_float(mirror16_u32(__float_as_uint(cs)));
   if (!live) return;
   const int tpg = gsum / 8;   // threads per group
   if (xsum != nullptr && g8 % tpg == 0) xsum[(size_t)t * (D / gsum) + g8 / tpg] = cs;
-  const int col = (8 * g8 & ~96) | block_at<BITS>((g8 >> 2) & 3) << 5, ch = col >> 7;   // the block's place
+  const int col = 8 * g8, ch = col >> 7, byte = col & 127;
   uint8_t* chunk = xp + ((size_t)t * (D / 128) + ch) * P3_ROWB;
-  if constexpr (BITS == 0) {
-    uint8_t* dst = chunk + (col & 127);
-    *reinterpret_cast<uint2*>(dst) = hi;
-    *reinterpret_cast<uint2*>(dst + 128) = lo;
-  } else if constexpr (BITS == 2) {   // even elements, then odd, four of each
-    uint8_t* dst = chunk + (col & 112) + (g8 & 1) * 4;
-    *reinterpret_cast<uint32_t*>(dst) = __builtin_amdgcn_perm(hi.y, hi.x, 0x06040200u);
-    *reinterpret_cast<uint32_t*>(dst + 8) = __builtin_amdgcn_perm(hi.y, hi.x, 0x07050301u);
-    *reinterpret_cast<uint32_t*>(dst + 128) = __builtin_amdgcn_perm(lo.y, lo.x, 0x06040200u);
-    *reinterpret_cast<uint32_t*>(dst + 136) = __builtin_amdgcn_perm(lo.y, lo.x, 0x07050301u);
-  } else if constexpr (BITS == PLANE_EVEN_ODD) {
-    uint8_t* dst = chunk + (col & 96) + (g8 & 3) * 4;
+  if constexpr (EVEN_ODD) {
+    uint8_t* dst = chunk + (byte & 96) + (g8 & 3) * 4;
     *reinterpret_cast<uint32_t*>(dst) = __builtin_amdgcn_perm(hi.y, hi.x, 0x06040200u);
     *reinterpret_cast<uint32_t*>(dst + 16) = __builtin_amdgcn_perm(hi.y, hi.x, 0x07050301u);
     *reinterpret_cast<uint32_t*>(dst + 128) = __builtin_amdgcn_perm(lo.y, lo.x, 0x06040200u);
     *reinterpret_cast<uint32_t*>(dst + 144) = __builtin_amdgcn_perm(lo.y, lo.x, 0x07050301u);
   } else {
-    uint8_t* dst = chunk + (col & 96);
-    const uint32_t hw[2] = {hi.x, hi.y}, lw[2] = {lo.x, lo.y};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      uint8_t* p = dst + plane_pos<BITS>((col & 31) + j);
-      p[0] = (uint8_t)(hw[j >> 2] >> (8 * (j & 3)));
-      p[128] = (uint8_t)(lw[j >> 2] >> (8 * (j & 3)));
-    }
+    *reinterpret_cast<uint2*>(chunk + byte) = hi;
+    *reinterpret_cast<uint2*>(chunk + 128 + byte) = lo;
   }
   if ((g8 & 3) == 0) {
     const uint32_t sc = (uint32_t)(E + 127) | ((uint32_t)(E + 123) << 8);
@@ -697,13 +677,13 @@ __global__ void __launch_bounds__(P3_THREADS) p3_kernel(MxArgs g, int slices) {
 
 // Workspace of the block-scaled prefill beyond the tile list: x planes [T][D/128][256]
 // and scales [T][sb(D)], h planes [rows][F_pad/128][256] and scales [rows][sb(F_pad)],
-// affine group sums of x [T][D / G] and of h [rows][128 / G per 128 columns], G >= 32.
+// affine group sums of x [T][D/64 or D/128] and of h [rows][2 or 1 per 128 columns].
 size_t prefill_mx_ws_bytes(int T, int k, int D, int F) {
   const size_t rows = (size_t)T * k;
   const int fch = (F + 127) / 128;
   auto a256 = [](size_t v) { return (v + 255) & ~size_t(255); };
   return a256((size_t)T * D * 2) + a256((size_t)T * scale_row_bytes(D)) + a256(rows * fch * P3_ROWB) +
-         a256(rows * scale_row_bytes(fch * 128)) + a256((size_t)T * (D / 32) * 4) + a256(rows * fch * 4 * 4 + 64);   // (64: a macro's sums past the last row)
+         a256(rows * scale_row_bytes(fch * 128)) + a256((size_t)T * (D / 64) * 4) + a256(rows * fch * 2 * 4);
 }
 
 // Shapes and slot layouts the kernels take.  Their B-scale loads read 16 bytes per
@@ -741,63 +721,36 @@ bool prefill_mx_q2_supported(int D, int F, const decode::Layout& L) {
 
 namespace {
 
-// The workspace regions and both launches' arguments, for groups of 128 / gpc.
-struct PrefillCall {
-  uint8_t *xp, *xs;
-  float* xsum;
-  int sbx, sbh, fch;
-  MxArgs gu, dn;
-};
-
-PrefillCall prefill_call(int T, const uint8_t* pool, const decode::Layout& L, const int32_t* slot_table,
-                         const int32_t* offsets, const int2* tiles, const int32_t* tiles_n, const int32_t* row_token,
-                         const int32_t* row_slot, const float* row_w, int D, int F, int k, float limit, uint8_t* ws,
-                         uint16_t* y) {
-  auto a256 = [](size_t v) { return (v + 255) & ~size_t(255); };
-  const size_t rows = (size_t)T * k;
-  PrefillCall c;
-  c.fch = (F + 127) / 128;
-  c.sbx = scale_row_bytes(D);
-  c.sbh = scale_row_bytes(c.fch * 128);
-  c.xp = ws;
-  c.xs = c.xp + a256((size_t)T * D * 2);
-  uint8_t* hp = c.xs + a256((size_t)T * c.sbx);
-  uint8_t* hs = hp + a256(rows * c.fch * P3_ROWB);
-  c.xsum = reinterpret_cast<float*>(hs + a256(rows * c.sbh));
-  float* hsum = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(c.xsum) + a256((size_t)T * (D / 32) * 4));
-  c.gu = MxArgs{c.xp, c.xs, c.sbx, D / 128, row_token, pool, L, slot_table, offsets, tiles, tiles_n, row_token,
-                row_slot, row_w, D, F, k, limit, hp, hs, c.sbh, c.fch, nullptr, c.xsum, hsum, nullptr};
-  c.dn = MxArgs{hp, hs, c.sbh, c.fch, nullptr, pool, L, slot_table, offsets, tiles, tiles_n, row_token, row_slot,
-                row_w, F, D, k, limit, nullptr, nullptr, 0, 0, y, hsum, nullptr, nullptr};
-  return c;
-}
-
-// x's planes, in element order BITS, with the sums of its groups of gsum (0: none).
-template <int BITS>
-int launch_x_planes_rows(const PrefillCall& c, const uint16_t* x, int T, int D, int gsum, hipStream_t s) {
-  const int64_t n8 = (int64_t)T * D / 8;
-  hipLaunchKernelGGL(x_planes_rows_kernel<BITS>, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, s, x, T, D, c.xp,
-                     c.xs, c.sbx, gsum ? c.xsum : nullptr, gsum ? gsum : 128);
-  return check_launch("x_planes_rows_kernel");
-}
-
 template <int AK>
 int launch_p3(const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L, const int32_t* slot_table,
               const int32_t* offsets, const int2* tiles, const int32_t* tiles_n, int max_tiles,
               const int32_t* row_token, const int32_t* row_slot, const float* row_w, int D, int F, int k, float limit,
               uint8_t* ws, uint16_t* y, hipStream_t s) {
-  const PrefillCall c = prefill_call(T, pool, L, slot_table, offsets, tiles, tiles_n, row_token, row_slot, row_w, D,
-                                     F, k, limit, ws, y);
+  auto a256 = [](size_t v) { return (v + 255) & ~size_t(255); };
+  const size_t rows = (size_t)T * k;
+  const int fch = (F + 127) / 128;
+  const int sbx = scale_row_bytes(D), sbh = scale_row_bytes(fch * 128);
+  uint8_t* xp = ws;
+  uint8_t* xs = xp + a256((size_t)T * D * 2);
+  uint8_t* hp = xs + a256((size_t)T * sbx);
+  uint8_t* hs = hp + a256(rows * fch * P3_ROWB);
+  float* xsum = reinterpret_cast<float*>(hs + a256(rows * sbh));
+  float* hsum = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(xsum) + a256((size_t)T * (D / 64) * 4));
   constexpr bool Q2 = ak_fold(AK);
   constexpr int GPC = ak_gpc(AK);
-  int rc = launch_x_planes_rows<p4_order(AK)>(c, x, T, D, Q2 ? 128 / GPC : 0, s);
+  const int64_t groups = (int64_t)T * D / 8;
+  hipLaunchKernelGGL(x_planes_rows_kernel<ak_even_odd(AK)>, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, x, T, D, xp, xs,
+                     sbx, Q2 ? xsum : nullptr, 128 / GPC);
+  int rc = check_launch("x_planes_rows_kernel");
   if (rc) return rc;
-  const MxArgs &gu = c.gu, &dn = c.dn;
-  const int sbx = c.sbx, sbh = c.sbh, fch = c.fch;
   const int tiles8 = (max_tiles + 7) / 8 * 8;
+  MxArgs gu{xp, xs, sbx, D / 128, row_token, pool, L, slot_table, offsets, tiles, tiles_n, row_token, row_slot,
+            row_w, D, F, k, limit, hp, hs, sbh, fch, nullptr, xsum, hsum};
   const int s_gu = (fch * 128) / (P3_WAVES * 32);   // h's padded columns, 128 per workgroup
   const size_t lds_gu = (size_t)P3_STAGES * P3_ABYTES + (size_t)P3_MT * (sbx + 16) +
                         (Q2 ? (size_t)P3_MT * (D / 128) * GPC * 4 : 0);
+  MxArgs dn{hp, hs, sbh, fch, nullptr, pool, L, slot_table, offsets, tiles, tiles_n, row_token, row_slot, row_w,
+            F, D, k, limit, nullptr, nullptr, 0, 0, y, hsum, nullptr};
   const int s_dn = (D + P3_WAVES * 64 - 1) / (P3_WAVES * 64);
   const size_t lds_dn = (size_t)P3_STAGES * P3_ABYTES + (size_t)P3_MT * (sbh + 16) +
                         (Q2 ? (size_t)P3_MT * fch * GPC * 4 : 0);
@@ -863,25 +816,6 @@ int launch_prefill_mx_aff(int bits, int group, const uint16_t* x, int T, const u
   CACHALOT_P3AFF(2, 64) CACHALOT_P3AFF(3, 64) CACHALOT_P3AFF(3, 128) CACHALOT_P3AFF(4, 64) CACHALOT_P3AFF(4, 128)
 #undef CACHALOT_P3AFF
   return fail(CACHALOT_EINVAL, "prefill (block-scaled): %d-bit codes in groups of %d", bits, group);
-}
-
-// Few rows per expert: x's planes in the bank's element order, then small_rows_mx.hip's
-// launches.  bits 0: FP4.  recs: the tiles of small_rows_mt(ak) rows (tile_recs_kernel).
-int small_rows_ak(int bits, int group) { return bits == 0 ? AK_FP4 : bits == 2 && group == 128 ? AK_Q2 : ak_aff(bits, group); }
-
-int launch_prefill_small(int bits, int group, const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
-                         const int4* recs, const int32_t* recs_n, const int32_t* row_token,
-                         const int32_t* row_slot, const float* row_w, int D, int F, int k, float limit, uint8_t* ws,
-                         uint16_t* y, hipStream_t s) {
-  PrefillCall c = prefill_call(T, pool, L, nullptr, nullptr, nullptr, recs_n, row_token, row_slot, row_w, D, F, k,
-                               limit, ws, y);
-  c.gu.recs = c.dn.recs = recs;
-  int rc;
-  if (bits == 2) rc = launch_x_planes_rows<2>(c, x, T, D, 32, s);
-  else if (bits == 3) rc = launch_x_planes_rows<3>(c, x, T, D, 32, s);
-  else rc = launch_x_planes_rows<0>(c, x, T, D, bits ? 32 : 0, s);
-  if (rc) return rc;
-  return launch_small_rows(small_rows_ak(bits, group), c.gu, c.dn, s);
 }
 
 }  // namespace cachalot

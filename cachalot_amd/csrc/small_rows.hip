@@ -1,12 +1,11 @@
 // Expert-major grouped experts with few rows per expert (batched decode, drafted
-// tokens, short prompts) on the gfx950 block-scaled matrix cores: every bank kind.
+// tokens, short prompts) as a weight stream on the bf16 matrix cores: every bank kind.
 //
 // Reference: affine_expert_forward_batched (src/cachalot/model/expert_affine.py:84-99),
 // routed_expert_forward_sgmm / _batched (fp4_sgmm_metal.py:318-333,
 // moe_prefill_batched.py:31-61), called per expert from moe_prefill_grouped.py:420-467.
 // Rounding points: g = bf16(x W1), u = bf16(x W3), h = bf16(silu(min(g, L)) * clip(u,
-// +-L) * w), y = bf16(h W2); the products accumulate in fp32.  Activations as two fp8
-// planes per 32-element block, as in prefill_mx.hip.
+// +-L) * w), y = bf16(h W2); the products accumulate in fp32.
 //
 // What bounds it: the weight bytes of the touched experts, each read once per tile of TPT
 // rows, so the kernel is a weight stream.  An item is 64 weight rows (gate/up: 32 of W1 and
@@ -14,19 +13,25 @@
 // workgroup take its macros of K (MC chunks of 128) in turn, so that at any time it reads
 // long contiguous runs of its rows.  (Waves owning 64 rows each, 256 per workgroup, read the
 // same bytes at 4.0 against 5.3 TB/s for FP4 at 24 tokens.)  A wave keeps its next macros'
-// codes in flight in registers, 16 bytes per lane and load; its share of the A planes (only
+// codes in flight in registers, 16 bytes per lane and load; its share of the A rows (only
 // the rows that exist) goes through an LDS ring of its own, so no wave waits for another
 // until the four partial sums meet in LDS, added in wave order.  The item's scales and
 // biases come as they lie, whole lines, one item ahead (4- and 8-byte loads per row and
-// macro made more requests than the codes: 2-bit 1370 against 1190 us per layer at 301
-// tokens, FP4 984 against 876 at 24).  The grid is what the chip holds at once, and a
+// macro made more requests than the codes).  The grid is what the chip holds at once, and a
 // workgroup takes an equal run of the items, its ring running on across them (one
 // workgroup per item: a third of the time goes to each one's start).
 //
-// Measured, two layers of D 4096 x F 2880, 384 experts top-6, router to combine: FP4, 24
-// tokens 1225 -> 864 us (362 + 243 -> 266 + 141 us per layer for the two kernels: 5.7 and
-// 5.4 TB/s); 3-bit g64, 7 tokens 1569 -> 430 us (536 + 229 -> 117 + 66).  The kernels before
-// are the 16-row bf16-MFMA ones of grouped.hip.
+// Operands.  x and h go in as the bf16 values they are and the codes as exact bf16, so
+// products are exact, the sums are the instruction's fp32 sums, and an infinity or a NaN
+// does what it does on the 16-row tiles of grouped.hip.  (Both as fp8 planes with fp4 codes
+// on the block-scaled instruction: an element 2^13 below its block's largest loses bits,
+// sums round at 2^-21 of their magnitudes, which turned one in twelve bf16 outputs against
+// one in a thousand, and E4M3 has no infinity.)
+//
+// Measured, kernel times per layer, gate/up + down, us: 16-row tiles -> planes -> here.
+// FP4, D 4096 x F 2880, 384 experts top-6, 24 tokens: 362 + 243 -> 256 + 135 -> 258 + 144
+// (5.7 and 5.1 TB/s).  3-bit g64, 5120 x 2304, 7 tokens: 536 + 229 -> 118 + 68 -> 128 + 72.
+// 2-bit g128, 5120 x 2304, 301 tokens: 798 + 367 as planes -> 826 + 445.
 //
 // A macro is two chunks of 2- or 4-bit codes (a load covers 32 or 64 contiguous bytes per
 // row and chunk) and four chunks of 3-bit codes: lane group kg then loads the whole of
@@ -34,68 +39,100 @@
 // lane-group swaps (v_permlane32_swap, v_permlane16_swap) hand each chunk's four 32-code
 // blocks to the four lane groups.  2-bit codes need two swaps: lane groups 0 and 1 hold
 // chunk 2q, 2 and 3 chunk 2q + 1, and exchange across the wave's halves, which gives lane
-// groups 0 .. 3 the blocks 0, 2, 1, 3 of the chunk; the planes store theirs in that order.
+// groups 0 .. 3 the blocks 0, 2, 1, 3 of the chunk (sr_block).
 //
-// The 16 A rows of an instruction.  A tile has TPT = 8 rows (4 in groups of 32); the
-// affine formula s * sum(x q) + b * sum(x) needs one dot product per group, and a chunk
-// holds GPC = 128 / G of them.  A row i is tile row i % TPT restricted to one group of the
-// chunk (zeros elsewhere) or, with one group per chunk, to one plane: rows 0 .. 7 the hi
-// plane, 8 .. 15 the lo plane, so one instruction does the work of two.  Result register
-// r of lane (j, kg) is A row 4 kg + r: its group or plane is a function of kg, so each
-// lane folds with one scale and one bias per weight row and chunk, acc = fma(s, d,
-// fma(b, sum x, acc)), and the lane groups' parts are summed once at the end.
-//
-// Codes as fp4 operands: 2-bit code q is the E2M1 encoding of q / 2 (column scale 2); 3-
-// and 4-bit codes are split, the low two bits so and the rest in a second instruction
-// (3-bit: bit 2 as the encoding of 2.0, the same scale; 4-bit: the high pair with scale 8).
-// (3-bit codes as six-bit E2M3 fields take one instruction and nine operations per 32
-// codes instead of 28, but the instruction sums fp8 x fp6 products, like fp8 x fp8 ones,
-// to 2^-19 of the sum of their magnitudes, against 2^-21 for fp8 x fp4.)  The order of a
-// block's 32 elements along K is free as long as A has the same, so each width uses the
-// order its codes spread to most cheaply (plane_pos): 2-bit codes are two masks per 16;
-// 3-bit codes leave three of every four on the nibble they reach by a shift of 0, 1 or 2
-// bits, and the fourth ones fill the fourth word (~55 operations in natural order).
+// The 16 A rows of an instruction.  Step q of a chunk takes codes 8 q .. + 7 of each lane
+// group's block, all four blocks at once.  A tile has TPT = 8 rows (4 in groups of 32 and for
+// 3-bit codes, whose four-chunk macros would leave room for one workgroup per CU); the affine
+// formula s * sum(x q) + b * sum(x) needs one dot product per group, and a chunk holds
+// GPC = 128 / G of them.  A row i is tile row i % TPT restricted to group (i / TPT) % GPC of
+// the chunk (zeros elsewhere).  Result register r of lane (j, kg) is A row 4 kg + r: its
+// group is a function of kg, so each lane folds with one scale and one bias per weight row
+// and chunk, acc = fma(s, d, fma(b, sum x, acc)), and the lane groups' parts are summed once
+// at the end.  The order of a block's 32 elements along K is free as long as A has the same,
+// so each width uses the order its codes spread to most cheaply (sr_pos, code_values).
 #include <algorithm>
+#include <type_traits>
 
 #include "decode_common.h"
 #include "mfma_tile.h"
-#include "mx_tile.h"
-#include "prefill_mx.h"
 
 namespace cachalot {
 namespace {
 
 using namespace decode;
-using namespace pmx;
+using tile::bf16x8_t;
+using tile::f32x4_t;
 
 constexpr int SR_THREADS = 256;
 constexpr int SR_WAVES = 4;
 constexpr int SR_FRAGS = 4;          // 16-row weight fragments per wave (NM * NF)
-constexpr uint32_t E8M0_EIGHT = 130u;
+constexpr int SR_ROWB = 256;         // one A row's chunk: 128 bf16
 
-constexpr int sr_tpt(int ak) { return ak_fold(ak) && (ak_gpc(ak) == 4 || ak_bits(ak) == 3) ? 4 : 8; }
+// Weight kinds: FP4, or (BITS << 8) | G for affine codes in groups of G.
+constexpr int SR_FP4 = 0;
+constexpr int sr_kind(int bits, int group) { return bits == 0 ? SR_FP4 : (bits << 8) | group; }
+constexpr int sr_bits(int sk) { return sk == SR_FP4 ? 4 : sk >> 8; }
+constexpr int sr_group(int sk) { return sk == SR_FP4 ? 128 : sk & 255; }
+constexpr int sr_tpt(int sk) { return sk != SR_FP4 && (sr_group(sk) == 32 || sr_bits(sk) == 3) ? 4 : 8; }
+
+// The order of a 32-element block of A (x and h of affine banks): the one its BITS-bit
+// codes leave the spread in (code_values).  2-bit: the even elements of each 16, then the
+// odd ones.  3-bit: the even elements, then the odd ones.  4-bit: elements 3j at place 2j,
+// 3j + 1 at 2j + 1, and of the elements 3j + 2 the first five at 23 + 2j, the others at
+// 22 + 2 (j - 5).  BITS 0 (FP4): natural.
+template <int BITS>
+__host__ __device__ inline int sr_pos(int n) {
+  if (BITS == 2) return (n & 16) + ((n & 1) ? 8 + ((n & 15) >> 1) : (n & 15) >> 1);
+  if (BITS == 3) return (n & 1) * 16 + (n >> 1);
+  if (BITS == 4) {
+    const int j = n / 3, r = n - 3 * j;
+    return r < 2 ? 2 * j + r : j < 5 ? 23 + 2 * j : 12 + 2 * j;
+  }
+  return n;
+}
+
+struct SrArgs {
+  const uint8_t* a;           // A rows, bf16 [source rows][kch * 128]
+  int kch;                    // 128-element chunks along K
+  const int32_t* a_gather;    // source row of a tile row (row_token) or null (the row itself)
+  const float* asum;          // affine: sums of 32 A elements [source rows][kch * 4]
+  const uint8_t* pool;
+  Layout L;
+  const int4* recs;           // the tiles: expert, first row, end row, slot
+  const int32_t* recs_n;
+  const int32_t* row_token;
+  const int32_t* row_slot;
+  const float* row_w;
+  int K;                      // real K (D or F)
+  int N;                      // weight rows per matrix (F or D)
+  int k;
+  float limit;
+  uint16_t* h;                // gate/up: [rows][hkch * 128], columns past F zero
+  int hkch;
+  float* hsum;                // gate/up, affine: sums of 32 of h [rows][hkch * 4]
+  uint16_t* y;                // down: [T, k, N]
+};
 
 template <int AK>
 struct Sr {
-  static constexpr bool FOLD = ak_fold(AK);
-  static constexpr int BITS = AK == AK_FP4 ? 4 : ak_bits(AK);
-  static constexpr int G = ak_group(AK);
-  static constexpr int GPC = ak_gpc(AK);
+  static constexpr bool FOLD = AK != SR_FP4;
+  static constexpr int BITS = sr_bits(AK);
+  static constexpr int G = sr_group(AK);
+  static constexpr int GPC = FOLD ? 128 / G : 1;           // groups per chunk
   static constexpr int TPT = sr_tpt(AK);                   // rows per tile
-  static constexpr int PS = GPC * TPT <= 8 ? 2 : 1;        // planes apart in the A rows (2) or one after the other
   static constexpr int MC = BITS == 3 ? 4 : 2;             // chunks per macro
   static constexpr int RD = BITS == 3 || (FOLD && BITS == 4) ? 2 : 3;   // macros in flight, the one computed included
   static constexpr int CW = BITS * MC;                     // code words per lane, fragment and macro
-  static constexpr int EX = FOLD ? MC : 1;                 // 16-byte loads of A scales (and sums) per macro
-  static constexpr int ROWB = MC * P3_ROWB;                // one A row's macro
+  static constexpr int EX = FOLD ? MC : 1;                 // 16-byte loads of A sums per macro
+  static constexpr int ROWB = MC * SR_ROWB;                // one A row's macro
   static constexpr int STAGE = TPT * ROWB;
   static constexpr int ZROW = GPC > 1 ? ROWB : 0;          // a row of zeros
-  // LDS: the waves' A rings, the zeros, per wave the macro's A scales [TPT][8 MC] and sums
-  // [MC GPC][TPT], and two items' weight scales (and biases) as stored.  A wave's partial
-  // sums (4 KiB) go into the ring stage it computed last, or have room of their own.
+  // LDS: the waves' A rings, the zeros, per wave the macro's sums [MC GPC][TPT], and two
+  // items' weight scales (and biases) as stored.  A wave's partial sums (4 KiB) go into
+  // the ring stage it computed last, or have room of their own.
   static constexpr int RING = SR_WAVES * RD * STAGE;
-  static constexpr int ASC = TPT * 8 * MC, SXS = FOLD ? MC * GPC * TPT * 4 : 0;
-  static constexpr int WAVE = ASC + SXS;
+  static constexpr int WAVE = FOLD ? MC * GPC * TPT * 4 : 0;
   static constexpr int PARTW = SR_FRAGS * 4 * 64 * 4;
   static constexpr bool PART_IN_RING = STAGE >= PARTW;
   static constexpr int PART = PART_IN_RING ? 0 : SR_WAVES * PARTW;
@@ -149,54 +186,65 @@ __device__ __forceinline__ void exchange_halves(uint32_t* w) {
   }
 }
 
-__device__ __forceinline__ i32x8_t op4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-  return i32x8_t{(int)a, (int)b, (int)c, (int)d, 0, 0, 0, 0};
+// The 32-element block of a chunk that lane group kg holds the codes of.
+template <int BITS>
+__device__ __forceinline__ int sr_block(int kg) {
+  return BITS == 2 && (kg == 1 || kg == 2) ? 3 - kg : kg;
 }
 
-__device__ __forceinline__ uint32_t bfi(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
-
-// The fp4 operands of a lane's 32 codes in the order of plane_pos<BITS>: code q as the
-// E2M1 encoding of q / 2, 3- and 4-bit codes split into their low two bits (lo) and the
-// rest (hi: bit 2 as the encoding 0100 = 2.0; the high pair of 4-bit codes as 2-bit codes).
+// A lane's 32 codes as exact bf16 integers in the order of sr_pos<BITS>, eight per MFMA
+// step.  2-bit: spread to nibbles, E2M1 q / 2, the pair converter with scale 2 (full
+// rate).  3- and 4-bit: spread to six-bit fields, E2M3 q / 8, the 32-value converter with
+// scale 8 (the time of 18 instructions).
 template <int BITS>
-__device__ __forceinline__ void code_operands(const uint32_t* w, i32x8_t& lo, i32x8_t& hi) {
-  constexpr uint32_t M = 0x33333333u;
+__device__ __forceinline__ void code_values(const uint32_t* w, bf16x8_t (&b)[4]) {
   if constexpr (BITS == 2) {
-    lo = op4(w[0] & M, (w[0] >> 2) & M, w[1] & M, (w[1] >> 2) & M);
-  } else if constexpr (BITS == 4) {
-    lo = op4(w[0] & M, w[1] & M, w[2] & M, w[3] & M);
-    hi = op4((w[0] >> 2) & M, (w[1] >> 2) & M, (w[2] >> 2) & M, (w[3] >> 2) & M);
+    constexpr uint32_t M = 0x33333333u;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) b[s] = tile::fp4_codes_to_b((s & 1 ? w[s >> 1] >> 2 : w[s >> 1]) & M, 2.0f);
   } else {
-    // codes 4t + r, r < 3, move up r bits to nibble 3t + r of the first three words
-    const uint32_t x0 = bfi(0x00F00F00u, w[0] << 2, bfi(0xF00F00F0u, w[0] << 1, w[0]));
-    const uint32_t x1 = bfi(0x0F00F00Fu, __builtin_amdgcn_alignbit(w[1], w[0], 30),
-                            bfi(0x00F00F00u, __builtin_amdgcn_alignbit(w[1], w[0], 31), w[1]));
-    const uint32_t x2 = bfi(0xF00F00F0u, __builtin_amdgcn_alignbit(w[2], w[1], 30),
-                            bfi(0x0F00F00Fu, __builtin_amdgcn_alignbit(w[2], w[1], 31), w[2]));
-    // codes 4t + 3 (bits 12t + 9) fill the fourth
-    const uint32_t x3 = bfi(0x0F000000u, w[2] >> 5,
-                            bfi(0x00F00F00u, w[2] << 3, bfi(0xF00F00F0u, w[1] << 3, w[0] >> 9)));
-    lo = op4(x0 & M, x1 & M, x2 & M, x3 & M);
-    constexpr uint32_t H = 0x44444444u;
-    hi = op4(x0 & H, x1 & H, x2 & H, x3 & H);
+    typedef uint32_t u32x6_t __attribute__((ext_vector_type(6)));
+    u32x6_t f;
+    if constexpr (BITS == 3) {
+      // every second code already lies alone in a six-bit field
+      constexpr uint32_t M0 = 0xC71C71C7u, M1 = 0x71C71C71u, M2 = 0x1C71C71Cu;
+      const uint32_t o0 = __builtin_amdgcn_alignbit(w[1], w[0], 3), o1 = __builtin_amdgcn_alignbit(w[2], w[1], 3);
+      f = u32x6_t{w[0] & M0, w[1] & M1, w[2] & M2, o0 & M0, o1 & M1, (w[2] >> 3) & M2};
+    } else {
+      // fields 2j (bit 12j): codes 3j, in place; fields 2j + 1: codes 3j + 1, two bits up;
+      // the last ten fields (bit 132 + 6k): codes 3j + 2, from bit 68 on in place, those
+      // below two bits up
+      constexpr uint32_t E0 = 0x0F00F00Fu, E1 = 0xF00F00F0u, E2 = 0x00F00F00u;   // words 0, 3; 1; 2
+      constexpr uint32_t O0 = 0xC03C03C0u, O1 = 0x03C03C03u, O2 = 0x3C03C03Cu;
+      const uint32_t s0 = w[0] << 2, s1 = __builtin_amdgcn_alignbit(w[1], w[0], 30);
+      const uint32_t s2 = __builtin_amdgcn_alignbit(w[2], w[1], 30), s3 = __builtin_amdgcn_alignbit(w[3], w[2], 30);
+      f = u32x6_t{(w[0] & E0) | (s0 & O0), (w[1] & E1) | (s1 & O1), (w[2] & E2) | (s2 & O2), (w[3] & E0) | (s3 & O0),
+                  (w[2] & 0xF00F00F0u) | (s0 & 0x03C03C00u) | (w[3] >> 30), (w[3] & E2) | (s1 & O2)};
+    }
+    typedef __attribute__((ext_vector_type(32))) __bf16 bf16x32_t;
+    const bf16x32_t v = __builtin_amdgcn_cvt_scalef32_pk32_bf16_fp6(f, 8.0f);
+    b[0] = __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, 6, 7);
+    b[1] = __builtin_shufflevector(v, v, 8, 9, 10, 11, 12, 13, 14, 15);
+    b[2] = __builtin_shufflevector(v, v, 16, 17, 18, 19, 20, 21, 22, 23);
+    b[3] = __builtin_shufflevector(v, v, 24, 25, 26, 27, 28, 29, 30, 31);
   }
 }
 
 // What a wave loads of one macro into registers, in this order (after its A rows).
 template <int AK>
 struct SrMacro {
-  uint4 ex[Sr<AK>::EX];                      // lanes 0 .. 7: A scales of row lane, 8 .. 15: sums of row lane - 8
+  uint4 ex[Sr<AK>::EX];                      // affine: the sums of A row lane (< TPT), four per chunk
   uint32_t codes[SR_FRAGS][Sr<AK>::CW];
 };
 
 // One workgroup takes a contiguous run of the items (tile, slice of 64 weight rows), an
 // equal share of them, so the grid is what the chip holds at once and all of it ends
 // together; the macros of its items are one sequence per wave, RD - 1 of them in flight
-// across the items' ends.  g.recs / g.tiles_n: the tiles.
+// across the items' ends.
 template <int AK, int NM, int NF>
-__global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices) {
+__global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(SrArgs g, int slices) {
   using S = Sr<AK>;
-  constexpr int TPT = S::TPT, MC = S::MC, GPC = S::GPC, G = S::G, BITS = S::BITS, PS = S::PS, RD = S::RD;
+  constexpr int TPT = S::TPT, MC = S::MC, GPC = S::GPC, G = S::G, BITS = S::BITS, RD = S::RD;
   static_assert(NM * NF == SR_FRAGS, "four fragments per wave");
   extern __shared__ __align__(16) uint8_t lds[];   // S::FIXED + 2 sr_scale_bytes
   const int tid = threadIdx.x;
@@ -206,14 +254,13 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
   // this workgroup's items; neighbouring runs on one XCD
   const int xcds = 8, per = gridDim.x / xcds;
   const int run = (int)(blockIdx.x % xcds) * per + (int)blockIdx.x / xcds;
-  const int64_t total = (int64_t)g.tiles_n[0] * slices;
+  const int64_t total = (int64_t)g.recs_n[0] * slices;
   const int it0 = (int)(total * run / gridDim.x), it1 = (int)(total * (run + 1) / gridDim.x);
   if (it0 >= it1) return;
 
   uint8_t* aring = lds + wave * RD * S::STAGE;
   uint8_t* zrow = lds + S::RING;
-  uint8_t* myas = zrow + S::ZROW + wave * S::WAVE;
-  float* mysx = reinterpret_cast<float*>(myas + S::ASC);
+  float* mysx = reinterpret_cast<float*>(zrow + S::ZROW + wave * S::WAVE);
   uint8_t* part0 = zrow + S::ZROW + SR_WAVES * S::WAVE;
   uint8_t* scales = part0 + S::PART;
   const int scb = sr_scale_bytes<AK>(g.K);
@@ -233,8 +280,6 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
   const uint8_t* base = g.pool;
   const uint8_t* asrc[NI];
   const uint8_t* exsrc = nullptr;
-  const bool ex_sum = S::FOLD && (lane & 8) != 0;
-  const int exstep = ex_sum ? 16 * MC : 8 * MC;
   int woff[SR_FRAGS];                                  // from the slot record (< 2^31: one expert)
   auto enter_item = [&]() {
     const int tile = i_item / slices, nw0 = (i_item - tile * slices) * WN;
@@ -251,11 +296,13 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
         const int r = q * RPI + lane / LPR;
         const int rr = row0 + min(r, i_rows - 1);
         const int src = g.a_gather ? g.a_gather[rr] : rr;
-        asrc[q] = g.ap + (size_t)src * nch * P3_ROWB + (((lane & 15) ^ (r & 15)) << 4);
+        asrc[q] = g.a + (size_t)src * nch * SR_ROWB + (((lane & 15) ^ (r & 15)) << 4);
       }
-      const int rr = row0 + min(lane & 7, i_rows - 1);
-      const int src = g.a_gather ? g.a_gather[rr] : rr;
-      exsrc = ex_sum ? reinterpret_cast<const uint8_t*>(g.asum + (size_t)src * nch * 4) : g.as + (size_t)src * g.sb;
+      if constexpr (S::FOLD) {
+        const int rr = row0 + min(lane & (TPT - 1), i_rows - 1);
+        const int src = g.a_gather ? g.a_gather[rr] : rr;
+        exsrc = reinterpret_cast<const uint8_t*>(g.asum + (size_t)src * nch * 4);
+      }
     }
 #pragma unroll
     for (int p = 0; p < SR_FRAGS; ++p)
@@ -283,10 +330,11 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
 #pragma unroll
     for (int q = 0; q < NI; ++q)
       if (q * RPI < i_rows)   // uniform: rows that do not exist are not read (their results are dropped)
-        tile::lds_load16_untracked(asrc[q] + (size_t)min(m * MC + achunk, nch - 1) * P3_ROWB, stage + q * 1024);
+        tile::lds_load16_untracked(asrc[q] + (size_t)min(m * MC + achunk, nch - 1) * SR_ROWB, stage + q * 1024);
+    if constexpr (S::FOLD) {
 #pragma unroll
-    for (int q = 0; q < S::EX; ++q)
-      out.ex[q] = *reinterpret_cast<const uint4*>(exsrc + m * exstep + 16 * (ex_sum ? q : min(q, MC / 2 - 1)));
+      for (int q = 0; q < MC; ++q) out.ex[q] = *reinterpret_cast<const uint4*>(exsrc + (m * MC + q) * 16);
+    }
 #pragma unroll
     for (int p = 0; p < SR_FRAGS; ++p) {
       if constexpr (BITS == 4) {
@@ -338,15 +386,14 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
 #pragma unroll
   for (int p = 0; p < SR_FRAGS; ++p) acc[p] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // the lane's A row: tile row i % TPT for the half of the chunk that lies in the row's
-  // group, the row of zeros for the other; with PS == 2 the upper rows carry the lo plane
-  const int at = i % TPT, ag = i / TPT % GPC, ap = PS == 2 ? i / (TPT * GPC) % 2 : 0;
-  const bool own0 = block_at<BITS>(kg >> 1) * 32 / G == ag, own1 = block_at<BITS>(2 + (kg >> 1)) * 32 / G == ag;
-  const int col0 = ((8 * ap + kg) ^ at) << 4, col1 = ((8 * ap + 4 + kg) ^ at) << 4;
-  const int col2 = ((8 + kg) ^ at) << 4, col3 = ((12 + kg) ^ at) << 4;
-  const uint8_t* sap = myas + at * (8 * MC) + ap;
+  // the lane's A row: tile row i % TPT where the lane's block lies in the row's group, the
+  // row of zeros elsewhere
+  const int at = i % TPT, blk = sr_block<BITS>(kg);
+  const bool own = blk * 32 / G == i / TPT % GPC;
+  int col[4];                                                  // 16-byte columns of the four steps
+#pragma unroll
+  for (int q = 0; q < 4; ++q) col[q] = ((4 * blk + q) ^ at) << 4;
   const int dg = (4 * kg) / TPT % GPC;                         // the group of the lane's results
-  const bool dlo = PS == 2 && (4 * kg) / (TPT * GPC) % 2 == 1; // they are the lo plane's (no bias term)
   const float* sxp = mysx + dg * TPT + (4 * kg) % TPT;
 
   // the partial sums of the waves meet; wave r finishes result register r
@@ -376,16 +423,16 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
       float t = 0.0f;
 #pragma unroll
       for (int w = 0; w < SR_WAVES; ++w) t = t + pw[w][p * 4 * 64];
-      // parts apart: rows [plane][group][row of the tile], four per lane group
-      if constexpr (TPT == 4 && GPC * PS >= 2) t = t + xor_f<16>(t);
-      if constexpr (GPC * PS * TPT == 16) t = t + xor_f<32>(t);
+      // groups apart: rows [group][row of the tile], four per lane group
+      if constexpr (TPT == 4 && GPC >= 2) t = t + xor_f<16>(t);
+      if constexpr (GPC * TPT == 16) t = t + xor_f<32>(t);
       sum[p] = c_slot >= 0 ? t : 0.0f;
     }
     ++c_item;   // (the barrier at the next item's first step frees the stages)
     if (tr >= c_rows || kg >= TPT / 4) return;   // the same in the 16 lanes of a row group
     if constexpr (NM == 2) {
-      float hv[NF];
-      float top = 0.0f;
+      uint16_t* dst = g.h + (size_t)c_prow * g.hkch * 128 + nw0;   // one 32-element block
+      float hsv = 0.0f;
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         float gv = round_bf16(sum[f]);
@@ -394,31 +441,11 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
           uv = fminf(fmaxf(uv, -g.limit), g.limit);
           gv = fminf(gv, g.limit);
         }
-        hv[f] = nw0 + 16 * f + i < g.N ? round_bf16((silu_f32(gv) * uv) * c_w) : 0.0f;
-        top = fmaxf(top, fabsf(hv[f]));
-      }
-      top = mx::row16_max(top);
-      const int E = plane_exp(top);
-      const float inv = __uint_as_float((uint32_t)(127 - E) << 23);
-      const int blk = (nw0 & ~127) / 32 + block_at<S::FOLD ? BITS : 0>((nw0 >> 5) & 3);   // the block's place
-      uint8_t* dst = g.hp + ((size_t)c_prow * g.hkch + (blk >> 2)) * P3_ROWB + (blk & 3) * 32;
-#pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        const float s = hv[f] * inv;
-        const uint32_t hi = mx::f32_to_e4m3(s);
-        const uint32_t lo = mx::f32_to_e4m3((s - mx::e4m3_to_f32(hi)) * 16.0f);
-        uint8_t* p = dst + plane_pos<S::FOLD ? BITS : 0>(16 * f + i);
-        p[0] = (uint8_t)hi;
-        p[128] = (uint8_t)lo;
-      }
-      if (i == 0) {
-        const uint32_t sc = (uint32_t)(E + 127) | ((uint32_t)(E + 123) << 8);
-        *reinterpret_cast<uint16_t*>(g.hs + (size_t)c_prow * g.hsb + blk * 2) = (uint16_t)sc;
+        const uint16_t hb = nw0 + 16 * f + i < g.N ? f32_to_bf16((silu_f32(gv) * uv) * c_w) : (uint16_t)0;
+        dst[sr_pos<S::FOLD ? BITS : 0>(16 * f + i)] = hb;
+        hsv = hsv + bf16_to_f32(hb);
       }
       if constexpr (S::FOLD) {   // the sum of the 32 h values (f, then the 16 lanes)
-        float hsv = 0.0f;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) hsv = hsv + hv[f];
         hsv = row16_sum(hsv);
         if (i == 0) g.hsum[(size_t)c_prow * g.hkch * 4 + nw0 / 32] = hsv;
       }
@@ -449,16 +476,13 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
       // an item's first step: every wave's quarter of its scales has landed too, and every
       // wave is past the partial sums of the item before
       if (c_j == 0) lds_sync();
-      if (lane < TPT) {
-#pragma unroll
-        for (int q = 0; q < MC / 2; ++q) *reinterpret_cast<uint4*>(myas + lane * (8 * MC) + 16 * q) = ring[v].ex[q];
-      } else if (S::FOLD && lane >= 8 && lane < 8 + TPT) {
+      if (S::FOLD && lane < TPT) {
 #pragma unroll
         for (int q = 0; q < S::EX; ++q) {   // four sums of 32 per chunk -> one per group; none past K
           const bool in = m * MC + q < nch;
           const float a = in ? __uint_as_float(ring[v].ex[q].x) : 0.0f, b = in ? __uint_as_float(ring[v].ex[q].y) : 0.0f;
           const float c = in ? __uint_as_float(ring[v].ex[q].z) : 0.0f, d = in ? __uint_as_float(ring[v].ex[q].w) : 0.0f;
-          float* o = mysx + q * GPC * TPT + (lane - 8);
+          float* o = mysx + q * GPC * TPT + lane;
           if constexpr (GPC == 1) {
             o[0] = (a + b) + (c + d);
           } else if constexpr (GPC == 2) {
@@ -482,92 +506,55 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
       }
       const uint8_t* sc = scales + (c_item & 1) * scb;
       const uint8_t* arow = aring + v * S::STAGE + at * S::ROWB;
-      const uint8_t* a0 = GPC == 1 || own0 ? arow : zrow;
-      const uint8_t* a1 = GPC == 1 || own1 ? arow : zrow;
+      const uint8_t* a0 = GPC == 1 || own ? arow : zrow;
 #pragma unroll
       for (int u = 0; u < MC; ++u) {
         const int c = m * MC + u;
         if (c >= nch) break;
         __builtin_amdgcn_sched_barrier(0);   // (chunks interleaved would spill)
-        const uint4 h0 = mx::lds16(a0 + u * P3_ROWB + col0);
-        const uint4 h1 = mx::lds16(a1 + u * P3_ROWB + col1);
-        const i32x8_t ahi = {(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
-        i32x8_t alo;
-        uint32_t sa;
-        if constexpr (PS == 1) {
-          const uint4 l0 = mx::lds16(a0 + u * P3_ROWB + col2);
-          const uint4 l1 = mx::lds16(a1 + u * P3_ROWB + col3);
-          alo = i32x8_t{(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
-          sa = (uint32_t)sap[(4 * u + kg) * 2] | ((uint32_t)sap[(4 * u + kg) * 2 + 1] << 8);
-        } else {
-          sa = sap[(4 * u + kg) * 2];
-        }
+        bf16x8_t a[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = tile::lds_a(a0, u * SR_ROWB + col[q]);
         if constexpr (!S::FOLD) {
-          const int blk = min(4 * c + kg, groups - 1);   // blocks past K meet zero A
-          uint32_t bs[SR_FRAGS];
-          i32x8_t b[SR_FRAGS];
+          const int eb = 4 * c + kg;                     // blocks past K meet zero A: any finite scale
+          float es[SR_FRAGS];
 #pragma unroll
-          for (int p = 0; p < SR_FRAGS; ++p) {
-            bs[p] = sc[(16 * p + i) * groups + blk];
-            const uint32_t* w = ring[v].codes[p] + 4 * u;
-            b[p] = op4(w[0], w[1], w[2], w[3]);
-          }
+          for (int p = 0; p < SR_FRAGS; ++p)
+            es[p] = e8m0_to_f32(eb < groups ? sc[(16 * p + i) * groups + eb] : 127u);
 #pragma unroll
-          for (int p = 0; p < SR_FRAGS; ++p) acc[p] = mx::mfma_fp8_fp4<0, true>(ahi, b[p], acc[p], sa, bs[p]);
-          if constexpr (PS == 1) {
-#pragma unroll
-            for (int p = 0; p < SR_FRAGS; ++p) acc[p] = mx::mfma_fp8_fp4<1, true>(alo, b[p], acc[p], sa, bs[p]);
-          }
-        } else {
-          const uint16_t* s16 = reinterpret_cast<const uint16_t*>(sc) + i * groups;
-          const int go = min(GPC * c + dg, groups - 1);   // groups past K meet zero A
-          float sw[SR_FRAGS];
-#pragma unroll
-          for (int p = 0; p < SR_FRAGS; ++p) sw[p] = scale_bits_to_f32(s16[16 * p * groups + go], g.L.f16);
-          constexpr uint32_t LS = mx::E8M0_TWO, HS = BITS == 4 ? E8M0_EIGHT : mx::E8M0_TWO;
-          f32x4_t d[SR_FRAGS];
-          // (two fragments at a time: all four's operands spill the 3-bit kernels)
-#pragma unroll
-          for (int pp = 0; pp < SR_FRAGS; pp += 2) {
-            i32x8_t lo[2], hi[2];
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-              code_operands<BITS>(ring[v].codes[pp + p] + BITS * u, lo[p], hi[p]);
-              d[pp + p] = mx::mfma_fp8_fp4<0, true>(ahi, lo[p], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, sa, LS);
-            }
-            if constexpr (PS == 1) {
-#pragma unroll
-              for (int p = 0; p < 2; ++p) d[pp + p] = mx::mfma_fp8_fp4<1, true>(alo, lo[p], d[pp + p], sa, LS);
-            }
-            if constexpr (BITS > 2) {
-#pragma unroll
-              for (int p = 0; p < 2; ++p) d[pp + p] = mx::mfma_fp8_fp4<0, true>(ahi, hi[p], d[pp + p], sa, HS);
-              if constexpr (PS == 1) {
-#pragma unroll
-                for (int p = 0; p < 2; ++p) d[pp + p] = mx::mfma_fp8_fp4<1, true>(alo, hi[p], d[pp + p], sa, HS);
-              }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          // the bias term: with the planes apart, the hi lanes take an even chunk's and the
-          // lo lanes the next one's
-          const bool bias_here = PS == 1 || u % 2 == 0;
-          if (bias_here) {
-            const int ub = PS == 1 ? u : u + (dlo ? 1 : 0);
-            const int gb = min(GPC * (m * MC + ub) + dg, groups - 1);
-            const float4 sx = *reinterpret_cast<const float4*>(sxp + ub * GPC * TPT);
-            const float sxv[4] = {sx.x, sx.y, sx.z, sx.w};
-#pragma unroll
-            for (int p = 0; p < SR_FRAGS; ++p) {
-              const float b = scale_bits_to_f32(s16[(64 + 16 * p) * groups + gb], g.L.f16);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) acc[p][r] = fmaf(sw[p], d[p][r], fmaf(b, sxv[r], acc[p][r]));
-            }
-          } else {
+          for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int p = 0; p < SR_FRAGS; ++p)
+              acc[p] = tile::mfma(a[q], tile::fp4_codes_to_b(ring[v].codes[p][4 * u + q], es[p]), acc[p]);
+        } else {
+          const uint16_t* s16 = reinterpret_cast<const uint16_t*>(sc) + i * groups;
+          const int go = min(GPC * c + dg, groups - 1);
+          const bool in = GPC == 1 || GPC * c + dg < groups;   // groups past K: nothing
+          const float4 sx = *reinterpret_cast<const float4*>(sxp + u * GPC * TPT);
+          const float sxv[4] = {sx.x, sx.y, sx.z, sx.w};
+          // (two fragments at a time, 3-bit one: more operands spill)
+          constexpr int FA = BITS == 3 ? 1 : 2;
 #pragma unroll
-              for (int r = 0; r < 4; ++r) acc[p][r] = fmaf(sw[p], d[p][r], acc[p][r]);
+          for (int pp = 0; pp < SR_FRAGS; pp += FA) {
+            bf16x8_t b[FA][4];
+            f32x4_t d[FA];
+#pragma unroll
+            for (int p = 0; p < FA; ++p) {
+              code_values<BITS>(ring[v].codes[pp + p] + BITS * u, b[p]);
+              d[p] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+              for (int p = 0; p < FA; ++p) d[p] = tile::mfma(a[q], b[p][q], d[p]);
+#pragma unroll
+            for (int p = 0; p < FA; ++p) {
+              const float sw = in ? scale_bits_to_f32(s16[16 * (pp + p) * groups + go], g.L.f16) : 0.0f;
+              const float bw = in ? scale_bits_to_f32(s16[(64 + 16 * (pp + p)) * groups + go], g.L.f16) : 0.0f;
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[pp + p][r] = fmaf(sw, d[p][r], fmaf(bw, sxv[r], acc[pp + p][r]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
           }
         }
       }
@@ -585,6 +572,37 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(MxArgs g, int slices)
   }
 }
 
+// x [T, D] -> rows in the order of sr_pos<BITS> and (sums != null) the sums of their
+// 32-element blocks.  One thread = 8 values.
+template <int BITS>
+__global__ void __launch_bounds__(256) sr_rows_kernel(const uint16_t* __restrict__ x, int64_t n,
+                                                      uint16_t* __restrict__ rows, float* __restrict__ sums) {
+  __shared__ __align__(16) uint16_t st[2048];
+  const int64_t at = (int64_t)blockIdx.x * 2048 + threadIdx.x * 8;
+  const uint4 v = *reinterpret_cast<const uint4*>(x + (at < n ? at : 0));
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint16_t b = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
+    const int e = threadIdx.x * 8 + j;
+    st[(e & ~31) + sr_pos<BITS>(e & 31)] = b;
+    s = s + bf16_to_f32(b);
+  }
+  s = s + __uint_as_float(xor1_u32(__float_as_uint(s)));
+  s = s + __uint_as_float(xor2_u32(__float_as_uint(s)));
+  __syncthreads();
+  if (at >= n) return;
+  *reinterpret_cast<uint4*>(rows + at) = *reinterpret_cast<const uint4*>(st + threadIdx.x * 8);
+  if (sums != nullptr && (threadIdx.x & 3) == 0) sums[at / 32] = s;
+}
+
+template <int BITS>
+int launch_sr_rows(const uint16_t* x, int64_t n, uint16_t* rows, float* sums, hipStream_t s) {
+  hipLaunchKernelGGL(sr_rows_kernel<BITS>, dim3((unsigned)((n + 2047) / 2048)), dim3(256), 0, s, x, n, rows, sums);
+  return check_launch("sr_rows_kernel");
+}
+
 template <int AK>
 struct SrLaunch {
   static size_t lds(int K) { return (size_t)Sr<AK>::FIXED + 2 * sr_scale_bytes<AK>(K); }
@@ -595,7 +613,7 @@ struct SrLaunch {
     return sr_steps(nmac, SR_WAVES - 1) >= Sr<AK>::RD - 1 && lds(K) <= 160 * 1024;
   }
   template <int NM, int NF>
-  static int go(const MxArgs& a, int slices, hipStream_t s) {
+  static int go(const SrArgs& a, int slices, hipStream_t s) {
     const size_t bytes = lds(a.K);
     auto k = sr_kernel<AK, NM, NF>;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -605,52 +623,91 @@ struct SrLaunch {
     hipLaunchKernelGGL(k, dim3(256 * per_cu), dim3(SR_THREADS), bytes, s, a, slices);
     return check_launch("sr_kernel");
   }
-  static int run(const MxArgs& gu, const MxArgs& dn, hipStream_t s) {
+  static int run(const SrArgs& gu, const SrArgs& dn, hipStream_t s) {
     if (int rc = go<2, 2>(gu, gu.hkch * 4, s)) return rc;   // 32 columns of h per item
     return go<1, 4>(dn, (dn.N + 63) / 64, s);
   }
 };
 
+// Workspace: x in the kind's order [T][D], its sums [T][D / 32], h [rows][F_pad], its sums
+// [rows][F_pad / 32] (64 bytes: a macro's sums past the last row).
+struct SrWs {
+  size_t x, xsum, h, hsum, total;
+};
+inline SrWs sr_ws(int T, int k, int D, int F) {
+  const size_t rows = (size_t)T * k, fpad = (size_t)(F + 127) / 128 * 128;
+  SrWs w;
+  w.x = 0;
+  w.xsum = w.x + align256((size_t)T * D * 2);
+  w.h = w.xsum + align256((size_t)T * (D / 32) * 4 + 64);
+  w.hsum = w.h + align256(rows * fpad * 2);
+  w.total = w.hsum + align256(rows * (fpad / 32) * 4 + 64);
+  return w;
+}
+
 }  // namespace
 
-// Rows per tile of a bank kind (the tile list's MT).
-int small_rows_mt(int ak) { return sr_tpt(ak); }
+size_t small_rows_ws_bytes(int T, int k, int D, int F) { return sr_ws(T, k, D, F).total; }
 
-template <int AK>
-static bool sr_fits(int D, int F) { return SrLaunch<AK>::fits(D) && SrLaunch<AK>::fits(F); }
+// Rows per tile of a bank kind (the tile list's MT); bits 0: FP4.
+int small_rows_mt(int bits, int group) { return sr_tpt(sr_kind(bits, group)); }
+
+// Calls go(integral constant SK) for the kind, or returns `otherwise`.
+template <typename R, typename Fn>
+static R sr_dispatch(int sk, R otherwise, Fn&& go) {
+#define CACHALOT_SR(K) \
+  if (sk == (K)) return go(std::integral_constant<int, (K)>());
+  CACHALOT_SR(SR_FP4)
+  CACHALOT_SR(sr_kind(2, 32)) CACHALOT_SR(sr_kind(2, 64)) CACHALOT_SR(sr_kind(2, 128))
+  CACHALOT_SR(sr_kind(3, 32)) CACHALOT_SR(sr_kind(3, 64)) CACHALOT_SR(sr_kind(3, 128))
+  CACHALOT_SR(sr_kind(4, 32)) CACHALOT_SR(sr_kind(4, 64)) CACHALOT_SR(sr_kind(4, 128))
+#undef CACHALOT_SR
+  return otherwise;
+}
 
 // A row's last chunk is read whole (2- and 3-bit codes): past a tensor's last row, where
-// the row is shorter, up to 47 bytes, which must still lie inside the slot record.
-bool small_rows_supported(int ak, int D, int F, const decode::Layout& L) {
+// the row is shorter, up to 36 bytes (3-bit, K = 128 n + 32), which must still lie inside
+// the slot record.
+bool small_rows_supported(int bits, int group, int D, int F, const decode::Layout& L) {
   if (!(D % 128 == 0 && D >= 128 && D <= 8192 && F % 32 == 0 && F >= 32 && F <= 8192)) return false;
-  const bool fold = ak_fold(ak);
-  const int bits = fold ? ak_bits(ak) : 4, group = ak_group(ak);
+  if (L.record_bytes > 0x7fffffff) return false;   // offsets inside a record are 32-bit
+  const bool fold = bits != 0;
   const int mats[3][3] = {{0, F, D}, {6, F, D}, {3, D, F}};   // w1, w3, w2: tensor, rows, K
   for (auto& m : mats) {
     const int64_t n = m[1], k = m[2], nch = (k + 127) / 128;
     const int64_t rb = fold ? (k + group - 1) / group * group * bits / 8 : k / 2;
-    const int64_t code_over = bits == 4 ? 0 : nch * 16 * bits - rb;
+    const int64_t code_over = bits == 4 || !fold ? 0 : nch * 16 * bits - rb;
     if (rb < 16 || L.off[m[0]] + n * rb + code_over > L.record_bytes) return false;
   }
-#define CACHALOT_SR(K) \
-  if (ak == (K)) return sr_fits<(K)>(D, F);
-  CACHALOT_SR(AK_FP4) CACHALOT_SR(AK_Q2)
-  CACHALOT_SR(ak_aff(2, 32)) CACHALOT_SR(ak_aff(2, 64))
-  CACHALOT_SR(ak_aff(3, 32)) CACHALOT_SR(ak_aff(3, 64)) CACHALOT_SR(ak_aff(3, 128))
-  CACHALOT_SR(ak_aff(4, 32)) CACHALOT_SR(ak_aff(4, 64)) CACHALOT_SR(ak_aff(4, 128))
-#undef CACHALOT_SR
-  return false;
+  return sr_dispatch(sr_kind(bits, group), false, [&](auto sk) {
+    return SrLaunch<decltype(sk)::value>::fits(D) && SrLaunch<decltype(sk)::value>::fits(F);
+  });
 }
 
-int launch_small_rows(int ak, const pmx::MxArgs& gu, const pmx::MxArgs& dn, hipStream_t s) {
-#define CACHALOT_SR(K) \
-  if (ak == (K)) return SrLaunch<(K)>::run(gu, dn, s);
-  CACHALOT_SR(AK_FP4) CACHALOT_SR(AK_Q2)
-  CACHALOT_SR(ak_aff(2, 32)) CACHALOT_SR(ak_aff(2, 64))
-  CACHALOT_SR(ak_aff(3, 32)) CACHALOT_SR(ak_aff(3, 64)) CACHALOT_SR(ak_aff(3, 128))
-  CACHALOT_SR(ak_aff(4, 32)) CACHALOT_SR(ak_aff(4, 64)) CACHALOT_SR(ak_aff(4, 128))
-#undef CACHALOT_SR
-  return fail(CACHALOT_EINVAL, "grouped experts (few rows): weight kind %d", ak);
+// recs: the tiles of small_rows_mt rows (tile_recs_kernel).
+int launch_small_rows(int bits, int group, const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
+                      const int4* recs, const int32_t* recs_n, const int32_t* row_token, const int32_t* row_slot,
+                      const float* row_w, int D, int F, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s) {
+  const SrWs w = sr_ws(T, k, D, F);
+  uint16_t* xr = reinterpret_cast<uint16_t*>(ws + w.x);
+  float* xsum = reinterpret_cast<float*>(ws + w.xsum);
+  float* hsum = reinterpret_cast<float*>(ws + w.hsum);
+  const int64_t n = (int64_t)T * D;
+  const uint16_t* a = xr;
+  int rc = CACHALOT_OK;
+  if (bits == 2) rc = launch_sr_rows<2>(x, n, xr, xsum, s);
+  else if (bits == 3) rc = launch_sr_rows<3>(x, n, xr, xsum, s);
+  else if (bits == 4) rc = launch_sr_rows<4>(x, n, xr, xsum, s);
+  else if (((uintptr_t)x & 15) != 0) rc = launch_sr_rows<0>(x, n, xr, nullptr, s);   // (LDS loads of 16 bytes)
+  else a = x;
+  if (rc) return rc;
+  const int fch = (F + 127) / 128;
+  const SrArgs gu{reinterpret_cast<const uint8_t*>(a), D / 128, row_token, xsum, pool, L, recs, recs_n, row_token,
+                  row_slot, row_w, D, F, k, limit, reinterpret_cast<uint16_t*>(ws + w.h), fch, hsum, nullptr};
+  const SrArgs dn{ws + w.h, fch, nullptr, hsum, pool, L, recs, recs_n, row_token,
+                  row_slot, row_w, F, D, k, limit, nullptr, 0, nullptr, y};
+  rc = sr_dispatch(sr_kind(bits, group), -1, [&](auto sk) { return SrLaunch<decltype(sk)::value>::run(gu, dn, s); });
+  return rc >= 0 ? rc : fail(CACHALOT_EINVAL, "grouped experts (few rows): %d-bit codes in groups of %d", bits, group);
 }
 
 }  // namespace cachalot

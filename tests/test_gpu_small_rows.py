@@ -1,4 +1,4 @@
-"""Grouped experts with few rows per expert (small_rows_mx.hip: the weight stream of batched decode,
+"""Grouped experts with few rows per expert (small_rows.hip: the weight stream of batched decode,
 drafted tokens and short prompts) against the oracle, every bank kind: experts of 1 .. 17 rows around
 the 4- and 8-row tile edges, an expert without a slot, dropped ids, K with partial chunks and groups,
 weight slices past F."""
@@ -63,3 +63,101 @@ def test_few_rows_per_expert(cuda, kind, d, f, monkeypatch):
         torch.cuda.synchronize()
         assert torch.equal(gout, out)
         grouped_experts(*args, **kw)
+
+
+KINDS = ["fp4", (2, 128, "bfloat16"), (2, 64, "float16"), (2, 32, "bfloat16"), (3, 128, "bfloat16"),
+         (3, 64, "float16"), (3, 32, "float16"), (4, 128, "float16"), (4, 64, "bfloat16"), (4, 32, "bfloat16")]
+
+
+def _bank(kind, d, f, E):
+    from cachalot_amd.storage.index import affine_format, fp4_format
+
+    fmt = fp4_format(d, f) if kind == "fp4" else affine_format(d, f, bits=kind[0], group_size=kind[1],
+                                                               scale_dtype=kind[2])
+    return fmt, make_store(fmt, n_layers=1, n_experts=E)
+
+
+def _two_per_expert(rng, E, device):
+    """E tokens, two routes each, every expert with two rows (2-bit: inside its range too)."""
+    idx = np.stack([rng.permutation(E), rng.permutation(E)], axis=1).astype(np.int32)
+    w = rng.dirichlet(np.ones(2), size=E).astype(np.float32)
+    return torch.from_numpy(idx).to(device), torch.from_numpy(w).to(device)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_strong_element_costs_its_neighbours_no_bits(cuda, kind):
+    """One element of every 32 is 2^15 times the others, and the codes (and biases) that meet it are
+    zero: the same bits as with that element zero, since bf16 operands carry each element by itself."""
+    from cachalot_amd.moe_prefill import grouped_experts
+
+    d, f, E = 2048, 1856, 32
+    fmt, store = _bank(kind, d, f, E)
+    pool = store.pool
+    rec = pool.storage.view(pool.n_slots, pool.record_bytes)
+    # code 5 of each 32: byte of the 32's run, bits kept
+    keep = {"fp4": [(2, 0x0F)], 2: [(1, 0xF3)], 3: [(1, 0x7F), (2, 0xFC)], 4: [(2, 0x0F)]}["fp4" if kind == "fp4" else kind[0]]
+    run = 16 if kind == "fp4" else 4 * kind[0]
+    for p in ("w1", "w3"):
+        o = pool.offsets[f"{p}.weight"]
+        codes = rec[:E, o:o + fmt.tensor_bytes(f"{p}.weight")].unflatten(1, (-1, run))
+        for byte, bits in keep:
+            codes[:, :, byte] &= bits
+        if kind != "fp4":
+            o = pool.offsets[f"{p}.biases"]
+            rec[:E, o:o + fmt.tensor_bytes(f"{p}.biases")] = 0
+    torch.cuda.synchronize()
+    idx, w = _two_per_expert(np.random.default_rng(5), E, cuda)
+    x = _bf16(osynth.activations(SEED, 5110, E, d), cuda)
+    strong, none = x.clone(), x.clone()
+    strong.view(E, -1, 32)[:, :, 5] = 2.0 ** 15
+    none.view(E, -1, 32)[:, :, 5] = 0.0
+    y = [grouped_experts(v, idx, w, pool, store.layer_table(0), want_terms=True)[2] for v in (strong, none)]
+    assert torch.equal(y[0].view(torch.int16), y[1].view(torch.int16))
+    assert y[1].float().abs().max() > 0
+
+
+@pytest.mark.parametrize("limit", [10.0, 0.0])
+@pytest.mark.parametrize("kind", KINDS)
+def test_infinities_and_nan_as_on_the_general_path(cuda, kind, limit, monkeypatch):
+    """A token with an infinity or a NaN: NaN, infinities and their signs where the 16-row tiles give
+    them; every other token keeps its bits."""
+    from cachalot_amd.moe_prefill import grouped_experts
+
+    d, f, E = 2048, 1856, 32
+    _, store = _bank(kind, d, f, E)
+    idx, w = _two_per_expert(np.random.default_rng(6), E, cuda)
+    x = _bf16(osynth.activations(SEED, 5111, E, d), cuda)
+
+    def run(v):
+        return grouped_experts(v, idx, w, store.pool, store.layer_table(0), swiglu_limit=limit, want_terms=True)[2]
+
+    finite = run(x)
+    for bad in (float("inf"), -float("inf"), float("nan")):
+        v = x.clone()
+        v[3, 100] = bad
+        v[9, d - 1] = bad
+        y = run(v)
+        monkeypatch.setenv("CACHALOT_GROUPED_SMALL", "1")
+        want = run(v)
+        monkeypatch.delenv("CACHALOT_GROUPED_SMALL")
+        for t in (3, 9):
+            for cls in (torch.isnan, torch.isposinf, torch.isneginf):
+                assert torch.equal(cls(y[t]), cls(want[t])), (kind, bad, cls.__name__)
+        rest = [t for t in range(E) if t not in (3, 9)]
+        assert torch.equal(y[rest].view(torch.int16), finite[rest].view(torch.int16)), (kind, bad)
+
+
+@pytest.mark.parametrize("kind", ["fp4", (2, 128, "bfloat16"), (3, 64, "float16")])
+def test_activations_off_the_16_byte_grid(cuda, kind):
+    from cachalot_amd.moe_prefill import grouped_experts
+
+    d, f, E = 2048, 1856, 32
+    _, store = _bank(kind, d, f, E)
+    idx, w = _two_per_expert(np.random.default_rng(7), E, cuda)
+    x = _bf16(osynth.activations(SEED, 5112, E, d), cuda)
+    flat = torch.empty(E * d + 4, dtype=torch.bfloat16, device=cuda)
+    off = flat[4:].view(E, d)
+    off.copy_(x)
+    assert off.data_ptr() % 16 == 8
+    y = [grouped_experts(v, idx, w, store.pool, store.layer_table(0), want_terms=True)[2] for v in (x, off)]
+    assert torch.equal(y[0].view(torch.int16), y[1].view(torch.int16))
