@@ -114,8 +114,8 @@ __global__ void __launch_bounds__(64) router_topk_kernel(const float* __restrict
 //
 // SP: the chunks are dealt to SP groups of 256 threads, a run of 64 / SP each (a subtree of
 // the pairwise sum), whose roots meet at the end.  What bounds the kernel is the fp32
-// multiply-adds, so it wants every SIMD busy: 64 tokens x 32 experts with SP = 1 does that
-// from some 2300 tokens on (768 workgroups at 4096 tokens x 384 experts), SP = 4 below.
+// multiply-adds, so it wants every SIMD busy: SP = 1 needs several workgroups per CU for
+// that, SP = 4 one.
 constexpr int RT_TB = 2;             // experts per thread (eq + 16 b)
 constexpr int RT_E = 16 * RT_TB;     // experts per workgroup
 constexpr int RT_MAXCH = 80;         // D / 64 <= 80 (D <= 5120)
@@ -125,9 +125,13 @@ constexpr int64_t RT_MIN_DOTS = 160 * 384;   // scores
 __host__ __device__ inline int rt_stride(int ch) { return ch * 2 + ((ch / 8) % 2 == 0 ? 16 : 32); }
 
 // Chunk c of a tile's x rows, then its W rows, as 16-byte items (rows past T / E:
-// clamped, unused), and the store of those items into a staged buffer.
+// clamped, unused), and the store of those items into a staged buffer (threads past the
+// last item carry it again).  Plain vectors and stores without a condition: as uint4 under
+// one, the items in flight went through scratch memory, each waited for (4096 tokens x 384
+// experts, unsplit: 321 us against 275 us).
+typedef uint32_t rt_item __attribute__((ext_vector_type(4)));
 template <int N, int TT>
-__device__ __forceinline__ void rt_load(uint4 (&v)[N], const uint16_t* __restrict__ x, const uint16_t* __restrict__ W,
+__device__ __forceinline__ void rt_load(rt_item (&v)[N], const uint16_t* __restrict__ x, const uint16_t* __restrict__ W,
                                         int T, int D, int E, int t0, int e0, int c, int tid, int items, int per_row) {
   const int ch = 8 * per_row;
 #pragma unroll
@@ -135,17 +139,17 @@ __device__ __forceinline__ void rt_load(uint4 (&v)[N], const uint16_t* __restric
     const int it = min(tid + 256 * j, items - 1);
     const int r = it / per_row, q = it - r * per_row;
     const uint16_t* src = r < TT ? x + (size_t)min(t0 + r, T - 1) * D : W + (size_t)min(e0 + r - TT, E - 1) * D;
-    v[j] = *reinterpret_cast<const uint4*>(src + c * ch + 8 * q);
+    v[j] = *reinterpret_cast<const rt_item*>(src + c * ch + 8 * q);
   }
 }
 
 template <int N>
-__device__ __forceinline__ void rt_store(uint8_t* buf, const uint4 (&v)[N], int tid, int items, int per_row, int S) {
+__device__ __forceinline__ void rt_store(uint8_t* buf, const rt_item (&v)[N], int tid, int items, int per_row, int S) {
 #pragma unroll
   for (int j = 0; j < N; ++j) {
-    const int it = tid + 256 * j;
+    const int it = min(tid + 256 * j, items - 1);
     const int r = it / per_row, q = it - r * per_row;
-    if (it < items) *reinterpret_cast<uint4*>(buf + r * S + 16 * q) = v[j];
+    *reinterpret_cast<rt_item*>(buf + r * S + 16 * q) = v[j];
   }
 }
 
@@ -174,7 +178,7 @@ __global__ void __launch_bounds__(256 * SP) router_tiled_kernel(const uint16_t* 
 
   float stk[LEV][TA * RT_TB];
   float node[TA * RT_TB];
-  uint4 v[MAXIT];
+  rt_item v[MAXIT];
   rt_load<MAXIT, TT>(v, x, W, T, D, E, t0, e0, c0, tid, items, per_row);
   rt_store(st, v, tid, items, per_row, S);
   __syncthreads();
@@ -295,20 +299,24 @@ static void launch_scores_tt(const uint16_t* x, const uint16_t* W, int T, int D,
 int launch_router_scores(const uint16_t* x, const uint16_t* W, int T, int D, int E, float gate_temp, int fn,
                          float* scores, hipStream_t s, const decode::RouteTail* tail, uint8_t* xplanes) {
   decode::RouteTail none{};
-  // The tiled kernel from RT_MIN_DOTS scores on (384 experts: 160 tokens; 200 tokens 91 us
-  // on the 4-token kernel against 56, 1000 tokens 417 against 127).  Below four chip-filling
-  // rounds of 32 x 32 tiles the chunks are split over four groups of threads; of 16, 32 and
-  // 64 tokens per tile the fewest rounds, weighed by what a round of each takes (52, 71 and
-  // 117 us at D = 4096), win (1500 tokens: 186 us with 32, 214 with 16, 242 with 64, 262
-  // unsplit; 4096: 324 unsplit, 381 with 32).
+  // The tiled kernel from RT_MIN_DOTS scores on (384 experts: 160 tokens, 74 us on the
+  // 4-token kernel against 44; 1000 tokens 410 against 95; with 8 experts, 4096 tokens, the
+  // same 48 us, 16384 tokens 166 against 110).  Of 16, 32 and 64 tokens per tile with the chunks
+  // split and 64 unsplit the one whose rounds of 256 workgroups take least, by what they
+  // take at D = 4096 (us, router and top-k, 384 experts: measured 16 / 32 / 64 / unsplit at
+  // 500 tokens 69 / 62 / 91 / 175, 1500: 149 / 163 / 173 / 193, 2049: 201 / 215 / 175 / 200, 4096:
+  // 341 / 319 / 260 / 275, 8192: 673 / 632 / 511 / 477).  Unsplit, up to four workgroups share a CU,
+  // and the first two of them cost little more than one.
   if ((int64_t)T * E >= RT_MIN_DOTS && D % 512 == 0 && D / CHUNKS <= RT_MAXCH) {
     const int et = (E + RT_E - 1) / RT_E;
     auto rounds = [&](int tokens) { return ((int64_t)((T + tokens - 1) / tokens) * et + 255) / 256; };
-    if (rounds(32) >= 4) return launch_tiled<4, 1>(x, W, T, D, E, gate_temp, fn, scores, s);
-    const int64_t c16 = 52 * rounds(16), c32 = 71 * rounds(32), c64 = 117 * rounds(64);
-    if (c16 <= c32 && c16 <= c64) return launch_tiled<1, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
-    if (c32 <= c64) return launch_tiled<2, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
-    return launch_tiled<4, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
+    const int64_t c16 = 26 * rounds(16) + 18, c32 = 52 * rounds(32) + 8, c64 = 84 * rounds(64) + 6;
+    const int64_t whole = std::max<int64_t>(176, 68 * rounds(64) + 70);
+    const int64_t least = std::min(std::min(c16, c32), std::min(c64, whole));
+    if (whole == least) return launch_tiled<4, 1>(x, W, T, D, E, gate_temp, fn, scores, s);
+    if (c64 == least) return launch_tiled<4, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
+    if (c32 == least) return launch_tiled<2, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
+    return launch_tiled<1, 4>(x, W, T, D, E, gate_temp, fn, scores, s);
   }
   // tokens per wave: 4 from 8 tokens on, 2 below (twice the waves for a small batch:
   // B = 4 68.4 against 70 us per batched step; at B = 32, 2 per wave lost 2.6 us)

@@ -13,7 +13,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("t,d,e,order", [(160, 4096, 384, "ascending"), (161, 5120, 384, "rank"),
                                          (337, 4096, 384, "ascending"), (673, 5120, 384, "rank"),
                                          (1000, 4096, 384, "ascending"), (1100, 1024, 65, "rank"),
-                                         (65, 512, 1000, "ascending"), (2337, 512, 384, "rank")])
+                                         (65, 512, 1000, "ascending"), (2337, 512, 384, "rank"),
+                                         (500, 512, 384, "rank"), (6001, 512, 384, "ascending"),
+                                         (60, 5120, 1024, "rank")])
 def test_tiles_give_the_same_bits(cuda, t, d, e, order):
     from cachalot_amd import synth
     from cachalot_amd.router import route_topk_rows
