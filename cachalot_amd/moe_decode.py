@@ -19,6 +19,7 @@ from .router import RouterResult
 from .storage.index import ExpertFormat
 
 _WORKSPACES: dict[tuple, torch.Tensor] = {}
+_OUTGROWN: list[torch.Tensor] = []      # earlier workspaces: a captured graph may hold their addresses
 
 
 def is_q2_g128(fmt: ExpertFormat) -> bool:
@@ -35,10 +36,15 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     preceded by an eager call of the same shape so that the workspace exists
     before capture.  A new workspace is zero-filled: the bf16-MFMA layer decode keeps
     a completion counter in its first bytes that must start at zero (every call
-    leaves it zero)."""
+    leaves it zero).  An outgrown workspace stays allocated, since graphs captured over
+    it go on using it; a new one is at least twice the size, so they add up to less
+    than it."""
     key = (device.index,)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
+        if ws is not None:
+            _OUTGROWN.append(ws)
+            nbytes = max(nbytes, 2 * ws.numel())
         ws = torch.zeros(max(nbytes, 1), dtype=torch.uint8, device=device)
         _WORKSPACES[key] = ws
     return ws

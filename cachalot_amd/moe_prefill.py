@@ -30,17 +30,6 @@ from .router import RouterResult, route_topk_batch, route_topk_rows
 from .shared_expert import shared_args, shared_expert_forward_batched
 from .storage.index import ExpertEntry
 
-_WORKSPACES: dict[int, torch.Tensor] = {}
-
-
-def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """Scratch for grouped calls, cached per device (grown on demand); calls sharing it must be ordered."""
-    ws = _WORKSPACES.get(device.index)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-        _WORKSPACES[device.index] = ws
-    return ws
-
 
 def permute(indices: torch.Tensor, weights: torch.Tensor, n_experts: int):
     """Routes [T, k] -> (offsets [E+1], row_token, row_slot, row_w) grouped by expert (device tensors)."""
@@ -102,7 +91,8 @@ def grouped_experts(x: torch.Tensor, indices: torch.Tensor, weights: torch.Tenso
         nbytes = L.cachalot_grouped_experts_affine_workspace_bytes(t, k, n_experts, d, f)
     else:
         nbytes = L.cachalot_grouped_experts_workspace_bytes(t, k, n_experts, d, f)
-    ws = _workspace(dev, nbytes)
+    # scratch of this call alone: the allocator keeps it on this stream and, under capture, in the graph's own pool
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     if generic:
         # 3- / 4-bit codes or groups of 32 / 64: the generic affine kernels (csrc/affine.hip)
         offsets, row_token, row_slot, row_w = permute(indices, weights, n_experts)

@@ -32,18 +32,6 @@ from . import _lib
 
 BLOCK = 32
 
-_WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
-
-
-def _workspace(device: torch.device, nbytes: int) -> torch.Tensor:
-    """Scratch per (device, stream): calls on one stream are ordered, calls on two streams may overlap."""
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
-    ws = _WORKSPACES.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-        _WORKSPACES[key] = ws
-    return ws
-
 
 def _bytes(w: torch.Tensor, name: str) -> torch.Tensor:
     if w.dtype == torch.float8_e4m3fn:
@@ -183,7 +171,8 @@ def _shared(x: torch.Tensor, w1, s1, w2, s2, w3, s3, swiglu_limit: float) -> tor
     y = torch.empty((m, d), dtype=torch.bfloat16, device=x.device)
     L = _lib.lib()
     nbytes = L.cachalot_shared_expert_fp8_workspace_bytes(m, d, f)
-    ws = _workspace(x.device, nbytes)
+    # scratch of this call alone: the allocator keeps it on this stream and, under capture, in the graph's own pool
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     rc = L.cachalot_shared_expert_fp8(x2.data_ptr(), w1.data_ptr(), s1.data_ptr(), w3.data_ptr(), s3.data_ptr(),
                                       w2.data_ptr(), s2.data_ptr(), m, d, f, float(swiglu_limit), y.data_ptr(),
                                       ws.data_ptr(), nbytes, _lib.stream_handle(x.device))

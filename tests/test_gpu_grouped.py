@@ -322,3 +322,79 @@ def test_one_expert_over_rows(cuda, kind):
     g = _np(got)
     assert np.array_equal(round_bf16(g), g)                 # each value a bf16 cast, as in the reference
     _check_rows(g, want, want[:, None, :], f"one expert, {kind}")
+
+
+def _other_stream(device, busy):
+    """A stream of its own whose queue holds `busy` large products."""
+    s = torch.cuda.Stream(device=device)
+    with torch.cuda.stream(s):
+        a = torch.zeros(4096, 4096, device=device)
+        for _ in range(busy):
+            a = a @ a
+    return s
+
+
+@pytest.mark.parametrize("kind", ["fp4", "q2", "q3"])
+def test_a_graph_keeps_its_scratch(cuda, kind):
+    """Captured over 16 tokens, then a larger eager call and fresh allocations: every replay gives the
+    eager output and leaves the other tensors alone."""
+    from cachalot_amd.moe_prefill import grouped_experts
+    from cachalot_amd.storage.index import affine_format, fp4_format
+
+    d, f, E, k = 1024, 1920, 16, 4
+    fmt = {"fp4": lambda: fp4_format(d, f), "q2": lambda: affine_format(d, f),
+           "q3": lambda: affine_format(d, f, bits=3, group_size=64, scale_dtype="float16")}[kind]()
+    store = make_store(fmt, n_layers=1, n_experts=E)
+    rng = np.random.default_rng(71)
+
+    def call(t):
+        x = _bf16(osynth.activations(SEED, 7100 + t, t, d), cuda)
+        idx = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(t)]).astype(np.int32)).to(cuda)
+        w = torch.from_numpy(rng.dirichlet(np.ones(k), size=t).astype(np.float32)).to(cuda)
+        return lambda: grouped_experts(x, idx, w, store.pool, store.layer_table(0))[1]
+
+    small, large = call(16), call(1500)
+    want = small()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = small()
+    large()
+    torch.cuda.synchronize()
+    fill = [torch.full((n,), 0x5A, dtype=torch.uint8, device=cuda) for n in [1 << 16] * 64 + [1 << 20] * 64 + [1 << 24] * 16]
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        large()
+    for t in fill:
+        assert bool((t == 0x5A).all())
+
+
+def test_two_streams_do_not_share_scratch(cuda):
+    """The same call on two streams at once: each gives its own output."""
+    from cachalot_amd.moe_prefill import grouped_experts
+    from cachalot_amd.storage.index import fp4_format
+
+    d, f, E, k, t = 2048, 1920, 16, 4, 24
+    store = make_store(fp4_format(d, f), n_layers=1, n_experts=E)
+    rng = np.random.default_rng(72)
+    args, want = [], []
+    for n in range(2):
+        x = _bf16(osynth.activations(SEED, 7200 + n, t, d), cuda)
+        idx = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(t)]).astype(np.int32)).to(cuda)
+        w = torch.from_numpy(rng.dirichlet(np.ones(k), size=t).astype(np.float32)).to(cuda)
+        args.append((x, idx, w, store.pool, store.layer_table(0)))
+        want.append(grouped_experts(*args[n])[1])
+    torch.cuda.synchronize()
+    streams = [_other_stream(cuda, 4) for _ in range(2)]   # both start late, together
+    got = [[], []]
+    for _ in range(20):
+        for n in range(2):
+            with torch.cuda.stream(streams[n]):
+                got[n].append(grouped_experts(*args[n])[1])
+    torch.cuda.synchronize()
+    for n in range(2):
+        for y in got[n]:
+            assert torch.equal(y, want[n])

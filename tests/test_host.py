@@ -256,3 +256,21 @@ def test_layout_carries_the_scale_dtype():
         assert HBMSlotPool(fmt, 1, device="cpu").layout().scale_dtype == code
     with pytest.raises(ValueError, match="bfloat16 or float16"):
         _lib.scale_dtype_code("float32")
+
+
+def test_an_outgrown_decode_workspace_stays_allocated(monkeypatch):
+    """A captured graph keeps the addresses of the workspace it was captured over."""
+    import weakref
+
+    import torch
+    from cachalot_amd import moe_decode
+
+    monkeypatch.setattr(moe_decode, "_WORKSPACES", {})
+    monkeypatch.setattr(moe_decode, "_OUTGROWN", [], raising=False)
+    cpu = torch.device("cpu")
+    held = [weakref.ref(moe_decode.workspace(cpu, n)) for n in (1000, 1001, 500_000, 500_001)]
+    assert all(r() is not None for r in held)
+    sizes = [r().numel() for r in held]
+    assert all(not r().any() for r in held)
+    assert moe_decode.workspace(cpu, 10) is held[-1]()
+    assert sum(sizes[:-1]) < sizes[-1]
