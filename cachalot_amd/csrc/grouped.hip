@@ -246,29 +246,51 @@ __global__ void __launch_bounds__(1024) tile_list_kernel(const int32_t* __restri
 }
 
 // The same tiles as records (expert, first row, end row, slot) for the few-row kernels.
+// With alt_mt they are taken only if they are at most num / den times as many as the other
+// kernels' tiles of alt_mt rows; else those are listed, and the list not taken is empty.
+struct AltTiles {
+  int mt, num, den;
+  int2* tiles;
+  int32_t* tiles_n;
+  uint32_t* zeros;
+};
 __global__ void __launch_bounds__(1024) tile_recs_kernel(const int32_t* __restrict__ offsets,
                                                          const int32_t* __restrict__ slot_table, int E, int MT,
-                                                         int4* __restrict__ recs, int32_t* __restrict__ recs_n) {
-  __shared__ int sc[1024];
+                                                         int4* __restrict__ recs, int32_t* __restrict__ recs_n,
+                                                         AltTiles alt) {
+  __shared__ int sc[1024], sa[1024];
   const int e = threadIdx.x;
-  int cnt = 0, r0 = 0, r1 = 0, slot = -1;
+  int cnt = 0, acnt = 0, r0 = 0, r1 = 0, slot = -1;
   if (e < E) {
     r0 = offsets[e];
     r1 = offsets[e + 1];
     slot = slot_table[e];
     cnt = r1 > r0 ? 1 + (r1 - r0 - 1) / MT : 0;
+    if (alt.mt) acnt = r1 > r0 ? 1 + (r1 - r0 - 1) / alt.mt : 0;
   }
   sc[e] = cnt;
+  sa[e] = acnt;
   __syncthreads();
   for (int off = 1; off < 1024; off *= 2) {
-    const int v = e >= off ? sc[e - off] : 0;
+    const int v = e >= off ? sc[e - off] : 0, va = e >= off ? sa[e - off] : 0;
     __syncthreads();
     sc[e] += v;
+    sa[e] += va;
     __syncthreads();
   }
-  const int first = sc[e] - cnt;
-  if (e == 1023) recs_n[0] = sc[1023];
-  for (int t = 0; t < cnt; ++t) recs[first + t] = make_int4(e, r0 + t * MT, min(r1, r0 + (t + 1) * MT), slot);
+  const bool few = alt.mt == 0 || (int64_t)sc[1023] * alt.den <= (int64_t)sa[1023] * alt.num;
+  if (e == 1023) {
+    recs_n[0] = few ? sc[1023] : 0;
+    if (alt.mt) alt.tiles_n[0] = few ? 0 : sa[1023];
+  }
+  if (few) {
+    const int first = sc[e] - cnt;
+    for (int t = 0; t < cnt; ++t) recs[first + t] = make_int4(e, r0 + t * MT, min(r1, r0 + (t + 1) * MT), slot);
+  } else {
+    if (e < ZERO_WORDS) alt.zeros[e] = 0u;
+    const int first = sa[e] - acnt;
+    for (int t = 0; t < acnt; ++t) alt.tiles[first + t] = make_int2(e, r0 + t * alt.mt);
+  }
 }
 
 // ------------------------------------------------------------ grouped GEMM ---
@@ -1001,23 +1023,24 @@ __global__ void __launch_bounds__(256) combine8_kernel(const uint16_t* __restric
   }
 }
 
-// Workspace of a grouped call: [tiles_n][tiles][hidden][x planes], 256-byte aligned regions.
+// Workspace of a grouped call: [tiles_n][tiles][recs][hidden][x planes][mx], 256-byte aligned
+// regions.  tiles_n: tile count, few-row record count at 64, zeros (g2_fp4_kernel) at 128.
+// tiles: int2, or one int4 record per active expert (matrix-core batched decode); recs: int4
+// records of the few-row kernels.
 // hidden: rows x F bf16, or rows x ceil(F / 128) plane blocks (matrix-core batched decode);
-// x planes: T x D / 128 plane blocks (same).
+// x planes: T x D / 128 plane blocks (same); mx: the regions of prefill_mx.hip or small_rows.hip.
 struct GroupedWs {
-  size_t tiles_n, tiles, hidden, xplanes, mx, total;
-  int max_tiles;
+  size_t tiles_n, tiles, recs, hidden, xplanes, mx, total;
 };
 
 inline GroupedWs grouped_ws(int T, int k, int E, int D, int F) {
   GroupedWs w;
   const int rows = T * k;
-  w.max_tiles = rows / 4 + std::min(E, rows) + 1;   // bound for MT >= 4
+  const size_t active = std::min(E, rows);
   w.tiles_n = 0;
   w.tiles = 256;
-  // int2 tiles, or int4 records (few-row kernels: one per tile; matrix-core batched decode:
-  // one per active expert)
-  w.hidden = w.tiles + align256((size_t)w.max_tiles * sizeof(int4));
+  w.recs = w.tiles + align256(std::max((rows / 16 + active + 1) * sizeof(int2), active * sizeof(int4)));
+  w.hidden = w.recs + align256((rows / 4 + active + 1) * sizeof(int4));   // (tiles of 4 rows at least)
   const size_t hid = std::max((size_t)rows * F * sizeof(uint16_t), (size_t)rows * ((F + 127) / 128) * 320);
   w.xplanes = w.hidden + align256(hid);
   w.mx = w.xplanes + align256((size_t)T * ((D + 127) / 128) * 320);
@@ -1075,6 +1098,21 @@ inline bool small_rows_wanted(int kind, int rows, int E) {
   if (kind == KIND_FP4) return rows < 5 * E;
   if (kind == KIND_Q2) return 2 * rows >= 3 * E && rows < 8 * E;
   return rows < 4 * E;
+}
+
+// Routes concentrated on a few experts (repeated tokens, padding, skew) leave the average
+// where it is but give the few-row kernel an expert's weights to read eight rows at a time
+// where the other kernels take 64 or 16; only the device knows, so both are launched and
+// one finds its list empty.  Taken: the few-row list where it is at most num / den times
+// the other: the time per tile of the two, which hardly depends on the routes (2-bit at 301
+// tokens 2.8 against 4.1 to 5.5 us, FP4 at 200 3.7 against 5).  Up to rows = 2 E (FP4) the
+// other kernels win nothing (100 tokens on 6 experts: 243 against 237 us); 2-bit below
+// 4 E and the other widths lose on them whatever the routes (160 tokens on 6 experts, 2-bit:
+// 365 against 1218; 3-bit, 200 tokens: 1159 against 1420).
+inline AltTiles small_rows_alt(int kind, int rows, int E, int mt) {
+  if (kind == KIND_Q2 && rows >= 4 * E) return {mt, 3, 2, nullptr, nullptr, nullptr};
+  if (kind == KIND_FP4 && rows >= 2 * E) return {mt, 7, 5, nullptr, nullptr, nullptr};
+  return {0, 0, 0, nullptr, nullptr, nullptr};
 }
 
 template <int KIND>
@@ -1135,48 +1173,49 @@ int launch_grouped(const uint16_t* x, const uint8_t* pool, const cachalot_expert
   hipLaunchKernelGGL(drop_zero_kernel, dim3(16), dim3(256), 0, s, offsets, E, T * k, T, k, D, row_token, row_slot, y);
   rc = check_launch("drop_zero_kernel");
   if (rc) return rc;
+  // the other kernels: 64-row tiles on the block-scaled matrix cores, FP4 128-row tiles, or
+  // the 64- / 16-row tiles here
+  int max_tiles = (T * k) / MT + std::min(E, T * k) + 1;
+  const bool mx = MT == 64 && !small_tiles_requested() && !prefill_bf16_requested() && max_tiles <= (1 << 20) &&
+                  (KIND == KIND_FP4  ? prefill_mx_supported(D, F, L)
+                   : KIND == KIND_Q2 ? prefill_mx_q2_supported(D, F, L)
+                                     : prefill_mx_aff_supported(SBITS, SGROUP, D, F, L));
+  const bool large = !mx && KIND == KIND_FP4 && MT == 64 && D % 128 == 0 && F % 32 == 0 &&
+                     !small_tiles_requested() && max_tiles <= (1 << 20);
+  const int tile_rows = mx ? prefill_mx_mt() : large ? G2_MT : MT;
   if (small) {
-    int4* recs = reinterpret_cast<int4*>(ws + wo.tiles);
-    hipLaunchKernelGGL(tile_recs_kernel, dim3(1), dim3(1024), 0, s, offsets, slot_table, E,
-                       small_rows_mt(SBITS, SGROUP), recs, tiles_n);
+    int4* recs = reinterpret_cast<int4*>(ws + wo.recs);
+    int32_t* recs_n = tiles_n + 16;
+    AltTiles alt = small_rows_alt(KIND, T * k, E, tile_rows);
+    alt.tiles = tiles;
+    alt.tiles_n = tiles_n;
+    alt.zeros = zeros;
+    const int tpt = small_rows_mt(SBITS, SGROUP);
+    hipLaunchKernelGGL(tile_recs_kernel, dim3(1), dim3(1024), 0, s, offsets, slot_table, E, tpt, recs, recs_n, alt);
     rc = check_launch("tile_recs_kernel");
     if (rc) return rc;
-    return launch_small_rows(SBITS, SGROUP, x, T, pool, L, recs, tiles_n, row_token, row_slot, row_w, D, F, k, limit,
-                             ws + wo.mx, y, s);
-  }
-  const int max_tiles = (T * k) / MT + std::min(E, T * k) + 1;
-  if (KIND == KIND_FP4 && MT == 64 && prefill_mx_supported(D, F, L) && !small_tiles_requested() &&
-      !prefill_bf16_requested() && max_tiles <= (1 << 20)) {
-    hipLaunchKernelGGL(tile_list_kernel, dim3(1), dim3(1024), 0, s, offsets, E, prefill_mx_mt(), tiles, tiles_n, zeros);
+    rc = launch_small_rows(SBITS, SGROUP, x, T, pool, L, recs, recs_n, row_token, row_slot, row_w, D, F, k, limit,
+                           ws + wo.mx, y, s);
+    if (rc || alt.mt == 0) return rc;
+    // taken only if n records > num / den n tiles, and there are at most rows / tpt +
+    // (tpt - 1) / tpt n records (n: at least the active experts)
+    max_tiles = std::min(max_tiles, alt.den * T * k / (tpt * alt.num - (tpt - 1) * alt.den) + 1);
+  } else {
+    hipLaunchKernelGGL(tile_list_kernel, dim3(1), dim3(1024), 0, s, offsets, E, tile_rows, tiles, tiles_n, zeros);
     rc = check_launch("tile_list_kernel");
     if (rc) return rc;
-    return launch_prefill_mx(x, T, pool, L, slot_table, offsets, tiles, tiles_n, max_tiles, row_token, row_slot,
-                             row_w, D, F, k, limit, ws + wo.mx, y, s);
   }
-  if (KIND == KIND_Q2 && MT == 64 && prefill_mx_q2_supported(D, F, L) && !small_tiles_requested() &&
-      !prefill_bf16_requested() && max_tiles <= (1 << 20)) {
-    // 2-bit g128 prefill on the block-scaled matrix cores (prefill_mx.hip)
-    hipLaunchKernelGGL(tile_list_kernel, dim3(1), dim3(1024), 0, s, offsets, E, prefill_mx_mt(), tiles, tiles_n, zeros);
-    rc = check_launch("tile_list_kernel");
-    if (rc) return rc;
-    return launch_prefill_mx_q2(x, T, pool, L, slot_table, offsets, tiles, tiles_n, max_tiles, row_token, row_slot,
-                                row_w, D, F, k, limit, ws + wo.mx, y, s);
+  if (mx) {
+    if constexpr (KIND == KIND_FP4)
+      return launch_prefill_mx(x, T, pool, L, slot_table, offsets, tiles, tiles_n, max_tiles, row_token, row_slot,
+                               row_w, D, F, k, limit, ws + wo.mx, y, s);
+    else if constexpr (KIND == KIND_Q2)
+      return launch_prefill_mx_q2(x, T, pool, L, slot_table, offsets, tiles, tiles_n, max_tiles, row_token, row_slot,
+                                  row_w, D, F, k, limit, ws + wo.mx, y, s);
+    else
+      return launch_prefill_mx_aff(SBITS, SGROUP, x, T, pool, L, slot_table, offsets, tiles, tiles_n, max_tiles,
+                                   row_token, row_slot, row_w, D, F, k, limit, ws + wo.mx, y, s);
   }
-  if (is_aff(KIND) && MT == 64 && prefill_mx_aff_supported(aff_bits(KIND), aff_group(KIND), D, F, L) &&
-      !small_tiles_requested() && !prefill_bf16_requested() && max_tiles <= (1 << 20)) {
-    // 2-bit g64, 3- and 4-bit g64 / g128 prefill on the block-scaled matrix cores
-    hipLaunchKernelGGL(tile_list_kernel, dim3(1), dim3(1024), 0, s, offsets, E, prefill_mx_mt(), tiles, tiles_n, zeros);
-    rc = check_launch("tile_list_kernel");
-    if (rc) return rc;
-    return launch_prefill_mx_aff(aff_bits(KIND), aff_group(KIND), x, T, pool, L, slot_table, offsets, tiles, tiles_n,
-                                 max_tiles, row_token, row_slot, row_w, D, F, k, limit, ws + wo.mx, y, s);
-  }
-  const bool large = KIND == KIND_FP4 && MT == 64 && D % 128 == 0 && F % 32 == 0 && !small_tiles_requested() &&
-                     max_tiles <= (1 << 20);
-  hipLaunchKernelGGL(tile_list_kernel, dim3(1), dim3(1024), 0, s, offsets, E, large ? G2_MT : MT, tiles, tiles_n,
-                     zeros);
-  rc = check_launch("tile_list_kernel");
-  if (rc) return rc;
   GroupedArgs gu{x, D, row_token, pool, L, slot_table, offsets, tiles, tiles_n, row_token, row_slot, row_w,
                  D, F, k, limit, hidden};
   GroupedArgs dn{hidden, F, nullptr, pool, L, slot_table, offsets, tiles, tiles_n, row_token, row_slot, row_w,

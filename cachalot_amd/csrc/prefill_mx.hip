@@ -125,7 +125,9 @@ __device__ __forceinline__ void encode8(const float (&v)[8], float inv, uint2& h
 template <bool EVEN_ODD>
 __global__ void __launch_bounds__(256) x_planes_rows_kernel(const uint16_t* __restrict__ x, int T, int D,
                                                             uint8_t* __restrict__ xp, uint8_t* __restrict__ xs,
-                                                            int sb, float* __restrict__ xsum, int gsum) {
+                                                            int sb, float* __restrict__ xsum, int gsum,
+                                                            const int32_t* __restrict__ tiles_n) {
+  if (tiles_n[0] == 0) return;   // (no tiles: nothing reads the planes)
   const int64_t t8 = (int64_t)blockIdx.x * 256 + threadIdx.x;   // index of an 8-value group
   const int per_row = D / 8;
   const bool live = t8 < (int64_t)T * per_row;
@@ -739,8 +741,8 @@ int launch_p3(const uint16_t* x, int T, const uint8_t* pool, const decode::Layou
   constexpr bool Q2 = ak_fold(AK);
   constexpr int GPC = ak_gpc(AK);
   const int64_t groups = (int64_t)T * D / 8;
-  hipLaunchKernelGGL(x_planes_rows_kernel<ak_even_odd(AK)>, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, x, T, D, xp, xs,
-                     sbx, Q2 ? xsum : nullptr, 128 / GPC);
+  hipLaunchKernelGGL(x_planes_rows_kernel<ak_even_odd(AK)>, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s,
+                     x, T, D, xp, xs, sbx, Q2 ? xsum : nullptr, 128 / GPC, tiles_n);
   int rc = check_launch("x_planes_rows_kernel");
   if (rc) return rc;
   const int tiles8 = (max_tiles + 7) / 8 * 8;

@@ -161,3 +161,32 @@ def test_activations_off_the_16_byte_grid(cuda, kind):
     assert off.data_ptr() % 16 == 8
     y = [grouped_experts(v, idx, w, store.pool, store.layer_table(0), want_terms=True)[2] for v in (x, off)]
     assert torch.equal(y[0].view(torch.int16), y[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("hot", [2, 5, 32])
+@pytest.mark.parametrize("kind,t", [("fp4", 40), ("fp4", 75), ((2, 128, "bfloat16"), 70), ((2, 128, "bfloat16"), 120)])
+def test_concentrated_and_spread_routes(cuda, kind, t, hot):
+    """The list of few-row tiles or, for routes on a few experts, of the other kernels' tiles, chosen on
+    the device: both against the oracle, and under capture each as the routes of its replay want it."""
+    from cachalot_amd.moe_prefill import grouped_experts
+
+    d, f, E, k = 2048, 1856, 32, 2
+    fmt, store = _bank(kind, d, f, E)
+    rng = np.random.default_rng(hot + t)
+    idx = np.stack([rng.permutation(hot)[:k] for _ in range(t)]).astype(np.int32)
+    w = rng.dirichlet(np.ones(k), size=t).astype(np.float32)
+    xb = osynth.activations(SEED, 5120 + t, t, d)
+    args = (_bf16(xb, cuda), torch.from_numpy(idx).to(cuda), torch.from_numpy(w).to(cuda), store.pool,
+            store.layer_table(0))
+    routed, out, y = grouped_experts(*args, want_routed=True, want_terms=True)
+    _grouped_check(f"{kind} {t} tokens on {hot} experts", fmt, 0, bf16_bits_to_f32(xb), idx, w, _np(routed), _f32(out),
+                   _f32(y), E)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        _, gout = grouped_experts(*args)
+    for n in (hot, 2, 32, hot):
+        args[1].copy_(torch.from_numpy(np.stack([rng.permutation(n)[:k] for _ in range(t)]).astype(np.int32)))
+        gout.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(gout, grouped_experts(*args)[1])
