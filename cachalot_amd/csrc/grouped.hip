@@ -1084,35 +1084,47 @@ inline bool prefill_bf16_requested() {
   return env && env[0] == '1';
 }
 
-// Where the few-row weight stream (small_rows.hip) is the faster one, in routes per
-// expert.  It reads an expert's weights once per 8 (4) rows, the 64-row tiles once per 64
-// but at a lower rate while tiles are nearly empty.  Per layer at D 4096 x F 2880, 384
-// experts top-6, against the path on the other side of the line, us:
-//   FP4: 200 tokens (3.1 per expert) 1366 against 1745 (bf16-MFMA 16-row tiles), 400
-//     (6.3) 1884 against 1752 (64-row tiles): up to 5;
-//   3-bit g64: 200 tokens 1940 against 5926 (bf16-MFMA), 256 2400 against 2190 (64-row, once
-//     its codes went in as fp6; 2650 before), 400 3300 against 2720 (before): up to 4, the same for the other widths and groups;
-//   2-bit g128: 64 tokens (1 per expert) 573 against 535 (one-token items per row), 128 (2)
-//     848 against 918, 400 1440 against 1703 (64-row), 600 (9.4) 2050 against 1850: 1.5 to 8.
+// Where the few-row weight stream (small_rows.hip) is taken, in routes per expert.  It reads
+// an expert's weights once per 8 (4) rows, the 64-row tiles once per 64 but at a lower rate
+// while tiles are nearly empty.  Per layer at D 4096 x F 2880, 384 experts top-6, spread
+// routes, few rows against the others, us:
+//   FP4: 64 tokens (1 per expert) 883 / 1191 (16-row bf16 tiles), 200 (3.1) 1391 / 1819, 256
+//     (4) 1468 / 1625 (64-row tiles), 320 (5) 1552 / 1652, 400 (6.3) 1707 / 1670: up to 5;
+//   2-bit g128: 96 tokens (1.5) 854 / 722 (batched decode), 128 (2) 980 / 897, 160 (2.5)
+//     1015 / 1064, 256 (4) 1184 / 1547 (64-row tiles), 500 (7.8) 1535 / 1590, 600 1624 / 1601:
+//     2.5 to 8;
+//   groups of 32, which have no 64-row kernel on the block-scaled matrix cores: 2-bit 200
+//     tokens 2288 / 5037 (16-row), 256 2677 / 12578 (64-row), 1200 (19) 9854 / 12902, 2000 (31)
+//     15946 / 13469; 3- and 4-bit alike: up to 32, the tiles counted (small_rows_alt);
+//   the other affine kinds: below 4, where the others are 16-row tiles (200 tokens: 3-bit g64
+//     1854 / 6201, 2-bit g64 1714 / 3736, 4-bit g64 1622 / 4092, 3-bit g128 1625 / 5986, 4-bit
+//     g128 1487 / 3843).  From 4 on the 64-row block-scaled kernels: 3-bit g64 2072 / 2257 at 4,
+//     2442 / 2260 at 4.7; the others cross between 7 and 10 for spread routes, but lose two-
+//     and threefold on concentrated ones.
 inline bool small_rows_wanted(int kind, int rows, int E) {
   if (kind == KIND_FP4) return rows < 5 * E;
-  if (kind == KIND_Q2) return 2 * rows >= 3 * E && rows < 8 * E;
+  if (kind == KIND_Q2) return 2 * rows >= 5 * E && rows < 8 * E;
+  if (is_aff(kind) && aff_group(kind) == 32) return rows < 32 * E;
   return rows < 4 * E;
 }
 
 // Routes concentrated on a few experts (repeated tokens, padding, skew) leave the average
-// where it is but give the few-row kernel an expert's weights to read eight rows at a time
+// where it is but give the few-row kernel an expert's weights to read 8 (4) rows at a time
 // where the other kernels take 64 or 16; only the device knows, so both are launched and
 // one finds its list empty.  Taken: the few-row list where it is at most num / den times
-// the other: the time per tile of the two, which hardly depends on the routes (2-bit at 301
-// tokens 2.8 against 4.1 to 5.5 us, FP4 at 200 3.7 against 5).  Up to rows = 2 E (FP4) the
-// other kernels win nothing (100 tokens on 6 experts: 243 against 237 us); 2-bit below
-// 4 E and the other widths lose on them whatever the routes (160 tokens on 6 experts, 2-bit:
-// 365 against 1218; 3-bit, 200 tokens: 1159 against 1420).
+// the other: the time per tile of the two, which hardly depends on the routes (2-bit g128
+// at 301 tokens 2.8 against 4.1 to 5.5 us, FP4 at 200 3.7 against 5, groups of 32 5 to 5.7
+// against 14 to 20 for 16 rows and 33 to 42 for 64).  FP4 below 2 E rows wins nothing on the
+// others (100 tokens on 6 experts: 243 against 237 us); the other kinds lose on them whatever
+// the routes (160 tokens on 6 experts, 2-bit g128: 365 against 1218; 200 tokens, 3-bit g64:
+// 1159 against 1420).
 inline AltTiles small_rows_alt(int kind, int rows, int E, int mt) {
-  if (kind == KIND_Q2 && rows >= 4 * E) return {mt, 3, 2, nullptr, nullptr, nullptr};
-  if (kind == KIND_FP4 && rows >= 2 * E) return {mt, 7, 5, nullptr, nullptr, nullptr};
-  return {0, 0, 0, nullptr, nullptr, nullptr};
+  AltTiles a{0, 0, 0, nullptr, nullptr, nullptr};
+  if (kind == KIND_Q2 && rows >= 4 * E) a = {mt, 3, 2, nullptr, nullptr, nullptr};
+  if (kind == KIND_FP4 && rows >= 2 * E) a = {mt, 7, 5, nullptr, nullptr, nullptr};
+  if (is_aff(kind) && aff_group(kind) == 32 && rows >= E)
+    a = rows >= 4 * E ? AltTiles{mt, 6, 1, nullptr, nullptr, nullptr} : AltTiles{mt, 5, 2, nullptr, nullptr, nullptr};
+  return a;
 }
 
 template <int KIND>

@@ -34,9 +34,12 @@ def test_few_rows_per_expert(cuda, kind, d, f, monkeypatch):
     monkeypatch.setenv("CACHALOT_PREFILL_BF16", "0")
     fmt = fp4_format(d, f) if kind == "fp4" else affine_format(d, f, bits=kind[0], group_size=kind[1],
                                                                scale_dtype=kind[2])
-    E, t, k = 32, 32, 2
+    E, k = 32, 2
     routes = [e for e, n in COUNTS.items() for _ in range(n)] + [LOST] * 5 + [-1, E, 1 << 20, -7, E + 3]
-    idx = np.asarray(routes, np.int32).reshape(k, t).T.copy()      # 64 routes: two per expert slot (2-bit: 1.5 to 8)
+    if kind[:2] == (2, 128):
+        routes += [17, 18] * 12                                    # 2.75 routes per expert slot (2.5 to 8 here)
+    t = len(routes) // k
+    idx = np.asarray(routes, np.int32).reshape(k, t).T.copy()      # 64 routes: two per expert slot
     rng = np.random.default_rng(d + f)
     idx = idx[rng.permutation(t)]
     w = rng.dirichlet(np.ones(k), size=t).astype(np.float32)
@@ -77,10 +80,10 @@ def _bank(kind, d, f, E):
     return fmt, make_store(fmt, n_layers=1, n_experts=E)
 
 
-def _two_per_expert(rng, E, device):
-    """E tokens, two routes each, every expert with two rows (2-bit: inside its range too)."""
-    idx = np.stack([rng.permutation(E), rng.permutation(E)], axis=1).astype(np.int32)
-    w = rng.dirichlet(np.ones(2), size=E).astype(np.float32)
+def _three_per_expert(rng, E, device):
+    """E tokens, three routes each, every expert with three rows (inside every kind's range)."""
+    idx = np.stack([rng.permutation(E) for _ in range(3)], axis=1).astype(np.int32)
+    w = rng.dirichlet(np.ones(3), size=E).astype(np.float32)
     return torch.from_numpy(idx).to(device), torch.from_numpy(w).to(device)
 
 
@@ -106,7 +109,7 @@ def test_a_strong_element_costs_its_neighbours_no_bits(cuda, kind):
             o = pool.offsets[f"{p}.biases"]
             rec[:E, o:o + fmt.tensor_bytes(f"{p}.biases")] = 0
     torch.cuda.synchronize()
-    idx, w = _two_per_expert(np.random.default_rng(5), E, cuda)
+    idx, w = _three_per_expert(np.random.default_rng(5), E, cuda)
     x = _bf16(osynth.activations(SEED, 5110, E, d), cuda)
     strong, none = x.clone(), x.clone()
     strong.view(E, -1, 32)[:, :, 5] = 2.0 ** 15
@@ -125,7 +128,7 @@ def test_infinities_and_nan_as_on_the_general_path(cuda, kind, limit, monkeypatc
 
     d, f, E = 2048, 1856, 32
     _, store = _bank(kind, d, f, E)
-    idx, w = _two_per_expert(np.random.default_rng(6), E, cuda)
+    idx, w = _three_per_expert(np.random.default_rng(6), E, cuda)
     x = _bf16(osynth.activations(SEED, 5111, E, d), cuda)
 
     def run(v):
@@ -153,7 +156,7 @@ def test_activations_off_the_16_byte_grid(cuda, kind):
 
     d, f, E = 2048, 1856, 32
     _, store = _bank(kind, d, f, E)
-    idx, w = _two_per_expert(np.random.default_rng(7), E, cuda)
+    idx, w = _three_per_expert(np.random.default_rng(7), E, cuda)
     x = _bf16(osynth.activations(SEED, 5112, E, d), cuda)
     flat = torch.empty(E * d + 4, dtype=torch.bfloat16, device=cuda)
     off = flat[4:].view(E, d)
@@ -164,7 +167,8 @@ def test_activations_off_the_16_byte_grid(cuda, kind):
 
 
 @pytest.mark.parametrize("hot", [2, 5, 32])
-@pytest.mark.parametrize("kind,t", [("fp4", 40), ("fp4", 75), ((2, 128, "bfloat16"), 70), ((2, 128, "bfloat16"), 120)])
+@pytest.mark.parametrize("kind,t", [("fp4", 40), ("fp4", 75), ((2, 128, "bfloat16"), 70), ((2, 128, "bfloat16"), 120),
+                                    ((2, 32, "bfloat16"), 30), ((3, 32, "float16"), 70), ((4, 32, "bfloat16"), 330)])
 def test_concentrated_and_spread_routes(cuda, kind, t, hot):
     """The list of few-row tiles or, for routes on a few experts, of the other kernels' tiles, chosen on
     the device: both against the oracle, and under capture each as the routes of its replay want it."""
