@@ -256,9 +256,9 @@ int launch_quant(const uint16_t* x, int ldx, int M, int K, bool swiglu, float li
 // not used), so that no branch makes the compiler wait for them.  Rows past M and N read
 // row 0 (masked at the store).  The products of an output are added block by
 // block in the order of K whatever the tile: all tiles give the same bits.
-// Measured (whole expert, D = 4096, F = 2880, M = 301 / 1000 / 4096): 168 / 177 / 446 us
+// Measured (whole expert, D = 4096, F = 2880, M = 301 / 1000 / 4096): 168 / 179 / 408 us
 // with 128 x 256 tiles of E4M3 in LDS, one block per stage and full fences; now
-// 68 / 130 / 408 us.  128 x 256 tiles with two blocks per stage 146 / 153 / 401 (one
+// 71 / 130 / 396 us.  128 x 256 tiles with two blocks per stage 146 / 153 / 401 (one
 // workgroup per CU), 64 x 256 tiles 106 / 166 / 552.
 
 // MI x NJ fragments per wave, 2 x 4 waves: a tile of 32 MI tokens x 64 NJ weight rows.
@@ -410,18 +410,19 @@ int launch_gemm(const LinearArgs& a, int nmat, hipStream_t s) {
 
 // Tile choice: token-tiled GEMV (one 16-token tile per workgroup, 8 chunks of
 // every wave in flight) for decode-sized M (M = 64: 46 us against 50 us for the GEMM
-// of smallest tiles at M = 65); above, the smallest of the LDS tiles that gives each of
-// the 256 CUs at most one workgroup: up to there a smaller tile only shortens what each
-// workgroup does, past it a second round costs more than it.  Whole expert in us,
-// 32 x 64 / 64 x 128 / 128 x 128 tiles throughout: D = 5120, F = 2304, M = 65 (216 and
-// 240 workgroups of 32 x 64) 42 / 67 / 93, M = 301 (180 and 200 of 64 x 128) 94 / 71 / 98,
-// M = 512 (288 and 320) 131 / 108 / 99; D = 4096, F = 2880, M = 128 (360 and 256 of
-// 32 x 64) 52 / 65 / 90, M = 768 (552 and 384 of 64 x 128) 183 / 135 / 128.
+// of smallest tiles at M = 65); above, the smallest of the LDS tiles whose grid the chip
+// takes in one round: a smaller tile only shortens what each workgroup does, past it a
+// second round costs more than it.  The light 32 x 64 tile runs two workgroups to a CU
+// beside each other (one GEMM in us, 32 x 64 / 64 x 128 / 128 x 128 tiles: K = 4096, N = 5760, M = 160,
+// 450 workgroups of 32 x 64, 36 / 39 / 52, M = 192, 540, 49 / 40 / 53; K = 5120, N = 4608, M = 224,
+// 504, 43 / 47 / 64, M = 256, 576, 58 / 47 / 63).  The heavier 64 x 128 one gains nothing from
+// a second (K = 5120, N = 4608, M = 448, 252 workgroups of it, 72 / 48 / 64, M = 512, 288, 89 / 73 / 64;
+// K = 2880, N = 4096, M = 512, 256, 47 / 33 / 41, M = 600, 320, 55 / 46 / 42).
 int launch_linear(const LinearArgs& a, int nmat, hipStream_t s) {
   if (a.M > 64) {
-    auto fits = [&](long tm, long tn) { return nmat * ((a.N + tn - 1) / tn) * ((a.M + tm - 1) / tm) <= 256; };
-    if (fits(32, 64)) return launch_gemm<1, 1, 4>(a, nmat, s);
-    if (fits(64, 128)) return launch_gemm<2, 2, 2>(a, nmat, s);
+    auto groups = [&](long tm, long tn) { return nmat * ((a.N + tn - 1) / tn) * ((a.M + tm - 1) / tm); };
+    if (groups(32, 64) <= 512) return launch_gemm<1, 1, 4>(a, nmat, s);
+    if (groups(64, 128) <= 256) return launch_gemm<2, 2, 2>(a, nmat, s);
     return launch_gemm<4, 2, 2>(a, nmat, s);
   }
   const dim3 grid((unsigned)(nmat * a.N / 16), (unsigned)((a.M + 15) / 16));

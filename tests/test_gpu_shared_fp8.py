@@ -101,7 +101,7 @@ def _one_ulp_of_exact(got, q, e, w, s):
 
 
 @pytest.mark.parametrize("m,k,n", [(65, 32, 64), (97, 160, 96), (1025, 96, 544), (1100, 352, 512), (2100, 96, 1120),
-                                   (2049, 224, 1088)])
+                                   (2049, 224, 1088), (1500, 352, 1088), (2049, 224, 544)])
 def test_fp8_linear_tiles_agree(cuda, m, k, n):
     """Each LDS tile of the many-token GEMM (32 x 64, 64 x 128, 128 x 128), ragged in tokens, rows and blocks per
     stage: the rows of a call in the smallest tile bit for bit (the products are added in one order), and those
