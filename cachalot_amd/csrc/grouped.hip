@@ -76,7 +76,7 @@ bool small_rows_supported(int bits, int group, int D, int F, const decode::Layou
 size_t small_rows_ws_bytes(int T, int k, int D, int F);
 int launch_small_rows(int bits, int group, const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
                       const int4* recs, const int32_t* recs_n, const int32_t* row_token, const int32_t* row_slot,
-                      const float* row_w, int D, int F, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s);
+                      const float* row_w, int D, int F, int E, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s);
 int launch_prefill_mx_q2(const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
                          const int32_t* slot_table, const int32_t* offsets, const int2* tiles,
                          const int32_t* tiles_n, int max_tiles, const int32_t* row_token, const int32_t* row_slot,
@@ -1206,8 +1206,8 @@ int launch_grouped(const uint16_t* x, const uint8_t* pool, const cachalot_expert
     hipLaunchKernelGGL(tile_recs_kernel, dim3(1), dim3(1024), 0, s, offsets, slot_table, E, tpt, recs, recs_n, alt);
     rc = check_launch("tile_recs_kernel");
     if (rc) return rc;
-    rc = launch_small_rows(SBITS, SGROUP, x, T, pool, L, recs, recs_n, row_token, row_slot, row_w, D, F, k, limit,
-                           ws + wo.mx, y, s);
+    rc = launch_small_rows(SBITS, SGROUP, x, T, pool, L, recs, recs_n, row_token, row_slot, row_w, D, F, E, k,
+                           limit, ws + wo.mx, y, s);
     if (rc || alt.mt == 0) return rc;
     // taken only if n records > num / den n tiles, and there are at most rows / tpt +
     // (tpt - 1) / tpt n records (n: at least the active experts)

@@ -17,9 +17,13 @@
 // the rows that exist) goes through an LDS ring of its own, so no wave waits for another
 // until the four partial sums meet in LDS, added in wave order.  The item's scales and
 // biases come as they lie, whole lines, one item ahead (4- and 8-byte loads per row and
-// macro made more requests than the codes).  The grid is what the chip holds at once, and a
-// workgroup takes an equal run of the items, its ring running on across them (one
-// workgroup per item: a third of the time goes to each one's start).
+// macro made more requests than the codes).  A workgroup takes an equal run of the items,
+// its ring running on across them (one workgroup per item: a third of the time goes to each
+// one's start).  The runs are as many as the chip holds at once, or up to SR_ROUNDS times
+// as many where each keeps SR_RUN items: with one round, a CU on which a kernel of another
+// stream (the shared expert) still held LDS when this one came took one workgroup for the
+// whole kernel, and the one left out ran after all others (2-bit, 301 tokens beside the
+// shared expert, gate/up 1092 against 826 us alone).
 //
 // Operands.  x and h go in as the bf16 values they are and the codes as exact bf16, so
 // products are exact, the sums are the instruction's fp32 sums, and an infinity or a NaN
@@ -30,7 +34,7 @@
 //
 // Measured, kernel times per layer, gate/up + down, us: 16-row tiles -> planes -> here.
 // FP4, D 4096 x F 2880, 384 experts top-6, 24 tokens: 362 + 243 -> 256 + 135 -> 258 + 144
-// (5.7 and 5.1 TB/s).  3-bit g64, 5120 x 2304, 7 tokens: 536 + 229 -> 118 + 68 -> 128 + 72.
+// (5.7 and 5.1 TB/s).  3-bit g64, 5120 x 2304, 7 tokens: 536 + 229 -> 118 + 68 -> 117 + 67.
 // 2-bit g128, 5120 x 2304, 301 tokens: 798 + 367 as planes -> 826 + 445.
 //
 // A macro is two chunks of 2- or 4-bit codes (a load covers 32 or 64 contiguous bytes per
@@ -139,6 +143,13 @@ struct Sr {
   static constexpr int FIXED = RING + ZROW + SR_WAVES * WAVE + PART;
   static_assert(WAVE % 16 == 0, "16-byte regions");
 };
+
+constexpr int SR_ROUNDS = 4, SR_RUN = 16;
+// Rounds of `slots` workgroups that `items` items are dealt to.
+__host__ __device__ inline int sr_rounds(int64_t items, int slots) {
+  const int64_t n = items / ((int64_t)slots * SR_RUN);
+  return n < 1 ? 1 : n < SR_ROUNDS ? (int)n : SR_ROUNDS;
+}
 
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 // A wave's macros are wave, wave + 4, ...: how many (at least one step, idle past the end).
@@ -256,11 +267,11 @@ struct SrMacro {
 };
 
 // One workgroup takes a contiguous run of the items (tile, slice of 64 weight rows), an
-// equal share of them, so the grid is what the chip holds at once and all of it ends
-// together; the macros of its items are one sequence per wave, RD - 1 of them in flight
-// across the items' ends.
+// equal share of them (slots: the workgroups the chip holds at once; the runs are a whole
+// number of rounds of them, so all of a round ends together); the macros of its items are
+// one sequence per wave, RD - 1 of them in flight across the items' ends.
 template <int AK, int NM, int NF>
-__global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(SrArgs g, int slices) {
+__global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(SrArgs g, int slices, int slots) {
   using S = Sr<AK>;
   constexpr int TPT = S::TPT, MC = S::MC, GPC = S::GPC, G = S::G, BITS = S::BITS, RD = S::RD;
   static_assert(NM * NF == SR_FRAGS, "four fragments per wave");
@@ -270,10 +281,12 @@ __global__ void __launch_bounds__(SR_THREADS, 2) sr_kernel(SrArgs g, int slices)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, kg = lane >> 4;
   // this workgroup's items; neighbouring runs on one XCD
-  const int xcds = 8, per = gridDim.x / xcds;
-  const int run = (int)(blockIdx.x % xcds) * per + (int)blockIdx.x / xcds;
   const int64_t total = (int64_t)g.recs_n[0] * slices;
-  const int it0 = (int)(total * run / gridDim.x), it1 = (int)(total * (run + 1) / gridDim.x);
+  const int runs = slots * sr_rounds(total, slots);
+  const int xcds = 8, per = runs / xcds;
+  const int run = (int)(blockIdx.x % xcds) * per + (int)blockIdx.x / xcds;
+  if ((int)blockIdx.x >= runs) return;
+  const int it0 = (int)(total * run / runs), it1 = (int)(total * (run + 1) / runs);
   if (it0 >= it1) return;
 
   uint8_t* aring = lds + wave * RD * S::STAGE;
@@ -632,20 +645,23 @@ struct SrLaunch {
     const int nmac = ((K + 127) / 128 + Sr<AK>::MC - 1) / Sr<AK>::MC;
     return sr_steps(nmac, SR_WAVES - 1) >= Sr<AK>::RD - 1 && lds(K) <= 160 * 1024;
   }
+  // max_tiles: at least the tiles there will be
   template <int NM, int NF>
-  static int go(const SrArgs& a, int slices, hipStream_t s) {
+  static int go(const SrArgs& a, int slices, int max_tiles, hipStream_t s) {
     const size_t bytes = lds(a.K);
     auto k = sr_kernel<AK, NM, NF>;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)bytes) != hipSuccess)
       return fail(CACHALOT_EHIP, "grouped experts (few rows): cannot grant %zu bytes of LDS", bytes);
-    const int per_cu = bytes <= 80 * 1024 ? 2 : 1;   // what each of the 256 CUs holds at once
-    hipLaunchKernelGGL(k, dim3(256 * per_cu), dim3(SR_THREADS), bytes, s, a, slices);
+    const int slots = 256 * (bytes <= 80 * 1024 ? 2 : 1);   // what the 256 CUs hold at once
+    const int grid = slots * sr_rounds((int64_t)max_tiles * slices, slots);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(SR_THREADS), bytes, s, a, slices, slots);
     return check_launch("sr_kernel");
   }
-  static int run(const SrArgs& gu, const SrArgs& dn, hipStream_t s) {
-    if (int rc = go<2, 2>(gu, gu.hkch * 4, s)) return rc;   // 32 columns of h per item
-    return go<1, 4>(dn, (dn.N + 63) / 64, s);
+  static int run(const SrArgs& gu, const SrArgs& dn, int rows, int E, hipStream_t s) {
+    const int max_tiles = rows / Sr<AK>::TPT + std::min(E, rows);
+    if (int rc = go<2, 2>(gu, gu.hkch * 4, max_tiles, s)) return rc;   // 32 columns of h per item
+    return go<1, 4>(dn, (dn.N + 63) / 64, max_tiles, s);
   }
 };
 
@@ -707,7 +723,7 @@ bool small_rows_supported(int bits, int group, int D, int F, const decode::Layou
 // recs: the tiles of small_rows_mt rows (tile_recs_kernel).
 int launch_small_rows(int bits, int group, const uint16_t* x, int T, const uint8_t* pool, const decode::Layout& L,
                       const int4* recs, const int32_t* recs_n, const int32_t* row_token, const int32_t* row_slot,
-                      const float* row_w, int D, int F, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s) {
+                      const float* row_w, int D, int F, int E, int k, float limit, uint8_t* ws, uint16_t* y, hipStream_t s) {
   const SrWs w = sr_ws(T, k, D, F);
   uint16_t* xr = reinterpret_cast<uint16_t*>(ws + w.x);
   float* xsum = reinterpret_cast<float*>(ws + w.xsum);
@@ -726,7 +742,7 @@ int launch_small_rows(int bits, int group, const uint16_t* x, int T, const uint8
                   row_slot, row_w, D, F, k, limit, reinterpret_cast<uint16_t*>(ws + w.h), fch, hsum, nullptr};
   const SrArgs dn{ws + w.h, fch, nullptr, hsum, pool, L, recs, recs_n, row_token,
                   row_slot, row_w, F, D, k, limit, nullptr, 0, nullptr, y};
-  rc = sr_dispatch(sr_kind(bits, group), -1, [&](auto sk) { return SrLaunch<decltype(sk)::value>::run(gu, dn, s); });
+  rc = sr_dispatch(sr_kind(bits, group), -1, [&](auto sk) { return SrLaunch<decltype(sk)::value>::run(gu, dn, T * k, E, s); });
   return rc >= 0 ? rc : fail(CACHALOT_EINVAL, "grouped experts (few rows): %d-bit codes in groups of %d", bits, group);
 }
 

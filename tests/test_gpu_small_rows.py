@@ -194,3 +194,24 @@ def test_concentrated_and_spread_routes(cuda, kind, t, hot):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(gout, grouped_experts(*args)[1])
+
+
+@pytest.mark.parametrize("kind", ["fp4", (3, 64, "float16"), (4, 32, "bfloat16")])
+def test_several_rounds_of_runs(cuda, kind):
+    """A call of more than 2 x 512 x 16 items, dealt in several rounds of runs: a token's terms are the
+    bits it gets in a call of few tokens (one round), whatever tiles and runs its rows fall into."""
+    from cachalot_amd.moe_prefill import grouped_experts
+
+    d, f, E, t, k = 2048, 2048, 320, 200, 4
+    _, store = _bank(kind, d, f, E)
+    rng = np.random.default_rng(11)
+    idx = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(t)]).astype(np.int32)).to(cuda)
+    w = torch.from_numpy(rng.dirichlet(np.ones(k), size=t).astype(np.float32)).to(cuda)
+    x = _bf16(osynth.activations(SEED, 5130, t, d), cuda)
+
+    def run(a, b):
+        return grouped_experts(x[a:b], idx[a:b], w[a:b], store.pool, store.layer_table(0), want_terms=True)[2]
+
+    whole = run(0, t)
+    parts = torch.cat([run(a, a + 8) for a in range(0, t, 8)])
+    assert torch.equal(whole.view(torch.int16), parts.view(torch.int16))
