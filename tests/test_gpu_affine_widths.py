@@ -103,10 +103,10 @@ def test_affine_decode_terms(cuda, bits, group, sd, path, monkeypatch):
     _check_decode(f"affine {bits}-bit g{group} {path} layer", fmt, 0, xf, oi[0], ow[0], _np(routed), _f32(out), terms, xf)
 
 
-# path: "mfma" = the default kernels (64-row tiles: the block-scaled prefill kernels for
-# 2-bit g64 and 3- / 4-bit g64 / g128, the bf16-MFMA grouped kernels for groups of 32;
-# 16-row tiles at t = 4), "bf16" = the bf16-MFMA grouped kernels (CACHALOT_PREFILL_BF16=1),
-# "valu" = the VALU kernels (CACHALOT_AFFINE_VALU=1)
+# path: "mfma" = the default kernels (from four routes per expert on the 64-row block-scaled
+# prefill kernels for 2-bit g64 and 3- / 4-bit g64 / g128; below, and for groups of 32, the
+# few-row kernels), "bf16" = the bf16-MFMA grouped kernels (CACHALOT_PREFILL_BF16=1; their 16-row
+# tiles and groups of 32: test_gpu_small_rows.py), "valu" = the VALU kernels (CACHALOT_AFFINE_VALU=1)
 GROUPED_CASES = [(3, 64, "float16", "mfma", 37, 16), (4, 32, "bfloat16", "mfma", 37, 16),
                  (3, 128, "bfloat16", "mfma", 37, 16), (2, 64, "float16", "mfma", 37, 16),
                  (4, 128, "float16", "mfma", 200, 8), (2, 32, "bfloat16", "mfma", 4, 16),

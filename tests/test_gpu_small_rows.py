@@ -25,17 +25,15 @@ CASES = [(kind, 2048, 1856) for kind in ("fp4", (2, 128, "bfloat16"), (2, 64, "f
 CASES += [("fp4", 5120, 2304), ((2, 128, "float16"), 4096, 2880), ((3, 64, "float16"), 4096, 2880)]
 
 
-@pytest.mark.parametrize("kind,d,f", CASES)
-def test_few_rows_per_expert(cuda, kind, d, f, monkeypatch):
+def _check_counts(cuda, what, kind, d, f, times=1):
+    """The routes of COUNTS (times over), a lost expert and dropped ids against the oracle, eager and captured."""
     from cachalot_amd.moe_prefill import grouped_experts
     from cachalot_amd.storage.index import affine_format, fp4_format
 
-    monkeypatch.setenv("CACHALOT_AFFINE_VALU", "0")
-    monkeypatch.setenv("CACHALOT_PREFILL_BF16", "0")
     fmt = fp4_format(d, f) if kind == "fp4" else affine_format(d, f, bits=kind[0], group_size=kind[1],
                                                                scale_dtype=kind[2])
     E, k = 32, 2
-    routes = [e for e, n in COUNTS.items() for _ in range(n)] + [LOST] * 5 + [-1, E, 1 << 20, -7, E + 3]
+    routes = [e for e, n in COUNTS.items() for _ in range(n * times)] + [LOST] * 5 + [-1, E, 1 << 20, -7, E + 3]
     if kind[:2] == (2, 128):
         routes += [17, 18] * 12                                    # 2.75 routes per expert slot (2.5 to 8 here)
     t = len(routes) // k
@@ -54,7 +52,7 @@ def test_few_rows_per_expert(cuda, kind, d, f, monkeypatch):
     gone = (idx < 0) | (idx >= E) | (idx == LOST)
     yf = _f32(y)
     assert not yf[gone].any()
-    _grouped_check(f"few rows {kind} D={d} F={f}", fmt, 0, bf16_bits_to_f32(xb), np.where(gone, -1, idx), w,
+    _grouped_check(f"{what} {kind} D={d} F={f}", fmt, 0, bf16_bits_to_f32(xb), np.where(gone, -1, idx), w,
                    _np(routed), _f32(out), yf, E, addend=bf16_bits_to_f32(ab))
     # the same under capture, replayed with other work in between
     g = torch.cuda.CUDAGraph()
@@ -66,6 +64,33 @@ def test_few_rows_per_expert(cuda, kind, d, f, monkeypatch):
         torch.cuda.synchronize()
         assert torch.equal(gout, out)
         grouped_experts(*args, **kw)
+
+
+@pytest.mark.parametrize("kind,d,f", CASES)
+def test_few_rows_per_expert(cuda, kind, d, f, monkeypatch):
+    monkeypatch.setenv("CACHALOT_AFFINE_VALU", "0")
+    monkeypatch.setenv("CACHALOT_PREFILL_BF16", "0")
+    _check_counts(cuda, "few rows", kind, d, f)
+
+
+# K of a few chunks: waves without a macro of their own (3- and 4-bit); FP4 and 2-bit codes, whose
+# rings are three macros deep, need K > 1792 in both projections and take the 16-row tiles here
+@pytest.mark.parametrize("kind,d,f", [(kind, d, f) for d, f in ((1024, 640), (128, 64))
+                                      for kind in ("fp4", (2, 64, "float16"), (2, 32, "bfloat16"),
+                                                   (3, 128, "bfloat16"), (3, 64, "float16"), (3, 32, "float16"),
+                                                   (4, 128, "float16"), (4, 64, "bfloat16"), (4, 32, "bfloat16"))])
+def test_few_rows_short_in_k(cuda, kind, d, f):
+    _check_counts(cuda, "few rows, short K", kind, d, f)
+
+
+# CACHALOT_PREFILL_BF16=1: two rows per expert slot the 16-row tiles, six the 64-row ones (FP4: 128-row)
+@pytest.mark.parametrize("times", [1, 3])
+@pytest.mark.parametrize("kind", ["fp4", (2, 64, "float16"), (2, 32, "bfloat16"), (3, 128, "bfloat16"),
+                                  (3, 64, "float16"), (3, 32, "float16"), (4, 128, "float16"), (4, 64, "bfloat16"),
+                                  (4, 32, "bfloat16")])
+def test_general_tiles(cuda, kind, times, monkeypatch):
+    monkeypatch.setenv("CACHALOT_PREFILL_BF16", "1")
+    _check_counts(cuda, f"general tiles x {times}", kind, 1024, 640, times)
 
 
 KINDS = ["fp4", (2, 128, "bfloat16"), (2, 64, "float16"), (2, 32, "bfloat16"), (3, 128, "bfloat16"),
