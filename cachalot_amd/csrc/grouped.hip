@@ -31,9 +31,12 @@
 // The grouped kernels also take the other affine widths (aff_kind<BITS, G>: 3- and
 // 4-bit codes, groups of 32 / 64 / 128, 2-bit codes in groups of 32 / 64), with the
 // codes read per step and the group formula applied per group (see chunk_mma_aff).
-// FP4, 2-bit g128 and (2-bit g64, 3- / 4-bit g64 / g128) affine prefill go to the
-// block-scaled kernels of prefill_mx.hip and prefill_affine_mx.hip; these kernels take
-// groups of 32, the other shapes and CACHALOT_PREFILL_BF16=1.
+// Few rows per expert go to small_rows.hip (every kind), chosen on the device against the
+// tiles here where routes may be concentrated; FP4, 2-bit g128 and (2-bit g64, 3- / 4-bit
+// g64 / g128) affine prefill to the block-scaled kernels of prefill_mx.hip and
+// prefill_affine_mx.hip; 2-bit g128 batches to decode_q2_mx.hip.  These kernels take what
+// is left: groups of 32 with many or concentrated rows, shapes too short in K for the
+// others, CACHALOT_PREFILL_BF16=1 and CACHALOT_GROUPED_SMALL=1.
 #include "decode_common.h"
 #include "mfma_tile.h"
 #include "permute_small.h"

@@ -245,9 +245,8 @@ int launch_quant(const uint16_t* x, int ldx, int M, int K, bool swiglu, float li
 // One 512-thread workgroup = a tile of TM tokens x TN rows of one matrix; wave (wm, wn),
 // wm < 2, wn < 4, owns MI x NJ fragments of 16 x 16.  K runs in stages of KB 32-element
 // blocks.  A thread converts what it staged to bf16 (scale folded in: exact) as it
-// writes it to LDS, so an element is converted once per workgroup: converted by each
-// wave that reads it (four waves read a row of A, two a row of B) the scaled
-// converters, a quarter of the VALU rate, were the bound.  KB blocks of a row are read by
+// writes it to LDS, so an element is converted once per workgroup and not by each wave
+// that reads it (four waves read a row of A, two a row of B).  KB blocks of a row are read by
 // consecutive lanes: 64 or 128 contiguous bytes a request, where one block at a time
 // asked L2 for every line four times.  LDS rows are 16 bytes longer than their blocks,
 // so the 16 rows of a fragment fall on distinct banks.  Two LDS stages, GM_RING stages

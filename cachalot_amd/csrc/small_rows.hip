@@ -32,10 +32,12 @@
 // sums round at 2^-21 of their magnitudes, which turned one in twelve bf16 outputs against
 // one in a thousand, and E4M3 has no infinity.)
 //
-// Measured, kernel times per layer, gate/up + down, us: 16-row tiles -> planes -> here.
-// FP4, D 4096 x F 2880, 384 experts top-6, 24 tokens: 362 + 243 -> 256 + 135 -> 258 + 144
-// (5.7 and 5.1 TB/s).  3-bit g64, 5120 x 2304, 7 tokens: 536 + 229 -> 118 + 68 -> 117 + 67.
-// 2-bit g128, 5120 x 2304, 301 tokens: 798 + 367 as planes -> 826 + 445.
+// Measured, kernel times per layer, gate/up + down, us, 384 experts top-6: 16-row tiles ->
+// planes -> here.  D 4096 x F 2880, FP4, 24 tokens: 362 + 243 -> 256 + 135 -> 258 + 144 (5.7 and
+// 5.1 TB/s); 3-bit g64, 7 tokens: 536 + 229 -> 117 + 64 -> 116 + 64.  5120 x 2304, 2-bit g128, 301
+// tokens beside the shared expert: 64-row tiles 1047 + 571 -> 748 to 938 + 370 -> 733 + 423 (VALU
+// 68 and 59 per cent busy, matrix cores 20 and 17: issue bound, where FP4 at 31 and 15 waits for
+// memory).
 //
 // A macro is two chunks of 2- or 4-bit codes (a load covers 32 or 64 contiguous bytes per
 // row and chunk) and four chunks of 3-bit codes: lane group kg then loads the whole of
